@@ -1236,6 +1236,17 @@ hipError_t dispatch(const int8_t* a, const void* w, const float* sa, const void*
                     int32_t* ws, int m, int n, int k, int schedule, hipStream_t stream) {
   const int cus = device_cu_count();
   int choice = schedule;
+  // Schedule 0 first weighs the ring kernel (gemm_ring.hip) against the others (gemm_choice,
+  // tile_plan.h); what it leaves goes by the rules below.
+  const bool persistent_ok =
+      !kWorkspace && n % 4 == 0 && reinterpret_cast<uintptr_t>(sw) % 8 == 0;
+  if (schedule == 0) {
+    const GemmChoice best = gemm_choice(m, n, k, cus, persistent_ok);
+    if (best.ring >= 0)
+      return launch_ring_gemm(best.ring, a, w, kCode, sa, sw, out, ws, m, n, k, stream);
+    if constexpr (!kWorkspace)
+      if (best.persistent) return launch_pp_gemm(a, w, kCode, sa, sw, out, m, n, k, stream);
+  }
   // Schedule 0 up to M = kSmallMaxM (tile_plan.h): the small-M kernel (gemm_small.hip), or
   // above kSmallOnlyMaxM 128 x 128 or 256 x 224 tiles where they finish sooner.
   if (schedule == 0 && m <= kSmallMaxM) {
@@ -1253,8 +1264,8 @@ hipError_t dispatch(const int8_t* a, const void* w, const float* sa, const void*
   // M = 16384, K = 17408, N = 5120: 5 rounds of 224-wide tiles and one of 160-wide beat 5
   // rounds of 256-wide; M = N = 4096: 2 rounds lose to 1).
   if constexpr (!kWorkspace) {
-    if (schedule == 0 && m >= 1024 && choice != 1 && n % 4 == 0 &&
-        reinterpret_cast<uintptr_t>(sw) % 8 == 0 && (choice == 4 || pp_beats_wide_tiles(m, n, cus)))
+    if (schedule == 0 && m >= 1024 && choice != 1 && persistent_ok &&
+        (choice == 4 || pp_beats_wide_tiles(m, n, cus)))
       return launch_pp_gemm(a, w, kCode, sa, sw, out, m, n, k, stream);
   }
   switch (choice) {

@@ -43,6 +43,12 @@ hipError_t launch_small_m_gemm(const int8_t* a, const void* w, WeightCode code, 
                                const void* sw, void* out, int32_t* workspace, int m, int n,
                                int k, int cus, hipStream_t stream);
 
+// Mid-size variant (gemm_ring.hip) with tile kRingTiles[tile] of tile_plan.h; identical
+// bits. Requires a and w 16-byte aligned; any n.
+hipError_t launch_ring_gemm(int tile, const int8_t* a, const void* w, WeightCode code,
+                            const float* sa, const void* sw, void* out, int32_t* workspace,
+                            int m, int n, int k, hipStream_t stream);
+
 // Large-M GEMM with two waves per SIMD (gemm_pp.hip), signed or biased UINT8 weights;
 // identical bits. Requires a and w 16-byte aligned, sw 8-byte aligned, n % 4 == 0.
 hipError_t launch_pp_gemm(const int8_t* a, const void* w, WeightCode code, const float* sa,

@@ -153,4 +153,81 @@ inline bool medium_tiles_pay(int m, int n, int cus) {
   return 2 * tiles224 < cus && tiles128 <= cus;
 }
 
+// Tiles of the ring kernel (gemm_mid.hip), each with the time of a round of them (one tile
+// on every CU): `fixed` + `per_k` * K / 1024 us. Fitted to 162 shapes measured on MI355X
+// (M = 17..3000 with (N, K) = 4096 x 4096, 17408 x 5120, 5120 x 17408, 7168 x 5120, 5120 x
+// 8704, 2048 x 8192, 1000 x 1024, 3000 x 2048 and 12000 x 3072; three rotated weight
+// copies): rms error 5%, and the kernel that the times below pick took 1.2% longer than the
+// best of all kernels in the mean. (64 x 80: 2.10 for a fitted 2.20; it is the faster one of
+// its size when the weights come from HBM, M = 256, N = 5120, K = 17408: 43.7 against 47.0 us.)
+struct RingTile {
+  int bm, bn;
+  double fixed, per_k;
+};
+constexpr RingTile kRingTiles[] = {
+    {32, 64, 2.2, 1.29},  {32, 96, 2.4, 1.71},  {64, 48, 2.6, 1.55},  {64, 64, 2.6, 1.72},
+    {64, 80, 3.2, 2.10},  {64, 96, 3.2, 2.23},  {64, 128, 3.5, 2.72}, {96, 96, 3.9, 2.71},
+    {128, 80, 4.2, 3.23}, {96, 128, 4.1, 3.42}, {128, 128, 4.9, 4.13}, {128, 160, 5.5, 4.93},
+    {192, 128, 6.2, 5.24}, {160, 160, 6.5, 5.42}, {192, 160, 6.9, 6.36}};
+constexpr int kRingTileCount = sizeof(kRingTiles) / sizeof(kRingTiles[0]);
+
+// Time (us) of one launch of a tiled GEMM that runs its tiles in rounds of one per CU: a
+// round of the other kernels' tiles by the same measurements (the persistent kernel's 256 x
+// 224 tiles; 256-wide tiles of the one-wave-per-SIMD kernel; the small-M kernel below). A
+// last round that is not full takes three quarters of a round plus its share of the rest
+// (fewer CUs share the caches and the power; the best single share over all tiles).
+constexpr double kLaunchTime = 1.5;
+inline double tiled_time(int64_t tiles, int cus, double fixed, double per_k, int k) {
+  const int64_t rest = tiles % cus;
+  const double rounds = double(tiles / cus) + (rest ? 0.75 + 0.25 * double(rest) / cus : 0.0);
+  return kLaunchTime + rounds * (fixed + per_k * k / 1024);
+}
+inline int64_t tile_count(int m, int n, int bm, int bn) {
+  return int64_t((m + bm - 1) / bm) * ((n + bn - 1) / bn);
+}
+inline double ring_time(const RingTile& t, int m, int n, int k, int cus) {
+  return tiled_time(tile_count(m, n, t.bm, t.bn), cus, t.fixed, t.per_k, k);
+}
+inline double persistent_time(int m, int n, int k, int cus) {
+  return tiled_time(tile_count(m, n, kPlanBM, kPlanBN), cus, 9.7, 8.56, k);
+}
+inline double wide_time(int m, int n, int bn, int k, int cus) {
+  return tiled_time(tile_count(m, n, kPlanBM, bn), cus, 9.7, 13.8 * bn / kPlanWideBN, k);
+}
+inline double small_time(int m, int n, int k, int cus) {
+  const SmallShape s = small_best_shape(m, n, cus);
+  const double rounds = double((tile_count(m, n, s.bm, s.bn) + cus - 1) / cus);
+  return kLaunchTime + rounds * (2.05 + 0.01146 * (s.bm + s.bn) * k / 1024);
+}
+
+// Schedule 0's first choice: the ring kernel with tile kRingTiles[ring] (ring >= 0), the
+// persistent kernel, or neither (the rules above). It goes by the times above: the ring
+// kernel is taken where its best tile is expected to beat the kernel that those rules take
+// (the small-M kernel up to kSmallMaxM, the persistent or the one-wave-per-SIMD kernel from
+// M = 1024 on) and the persistent kernel. The persistent kernel is also taken below M =
+// 1024 where its 256 x 224 tiles fill most of a round. persistent_ok: it can run this call.
+struct GemmChoice {
+  int ring;
+  bool persistent;
+};
+inline GemmChoice gemm_choice(int m, int n, int k, int cus, bool persistent_ok) {
+  GemmChoice choice{-1, false};
+  if (cus <= 0) return choice;
+  double best = 0.0;
+  for (int i = 0; i < kRingTileCount; ++i) {
+    const double t = ring_time(kRingTiles[i], m, n, k, cus);
+    if (choice.ring < 0 || t < best) best = t, choice.ring = i;
+  }
+  if (m <= kSmallMaxM && small_time(m, n, k, cus) <= best) return {-1, false};
+  if (m <= kSmallOnlyMaxM) return choice;
+  if (persistent_ok) {
+    if (m >= 1024 && !pp_beats_wide_tiles(m, n, cus))
+      return wide_time(m, n, kPlanWideBN, k, cus) <= best ? GemmChoice{-1, false} : choice;
+    return persistent_time(m, n, k, cus) <= best ? GemmChoice{-1, true} : choice;
+  }
+  const int wide = wide_tiles_pay(m, n, cus) ? kPlanWideBN : kPlanBN;
+  if (m >= 1024 && wide_time(m, n, wide, k, cus) <= best) return {-1, false};
+  return choice;
+}
+
 }  // namespace ci8

@@ -1,0 +1,84 @@
+"""Schedule 0's choice between the ring kernel and the others (gemm_choice in
+csrc/tile_plan.h), compiled on the CPU with g++: every ring tile is picked by one of the
+shapes that tests/test_gpu_ring.py runs on the GPU, and shapes worked out by hand from the
+round times go where they should."""
+
+import shutil
+import subprocess
+
+import pytest
+
+from tests.conftest import PKG
+from tests.test_gpu_ring import SHAPES
+
+PROGRAM = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "tile_plan.h"
+using namespace ci8;
+int main(int argc, char** argv) {
+  for (int i = 1; i + 4 < argc; i += 5) {
+    const GemmChoice c = gemm_choice(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]),
+                                     atoi(argv[i + 3]), atoi(argv[i + 4]) != 0);
+    std::printf("%d %d %d\n", c.ring < 0 ? 0 : kRingTiles[c.ring].bm,
+                c.ring < 0 ? 0 : kRingTiles[c.ring].bn, int(c.persistent));
+  }
+  std::printf("%d\n", kRingTileCount);
+  return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def choose(tmp_path_factory):
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("g++ not available")
+    folder = tmp_path_factory.mktemp("ring_plan")
+    (folder / "plan.cpp").write_text(PROGRAM)
+    subprocess.run([gxx, "-std=c++17", "-O1", f"-I{PKG / 'csrc'}", str(folder / "plan.cpp"), "-o",
+                    str(folder / "plan")], check=True)
+
+    def run(cases):
+        args = [str(int(v)) for case in cases for v in case]
+        lines = subprocess.run([str(folder / "plan"), *args], check=True, capture_output=True,
+                               text=True).stdout.split("\n")
+        return [tuple(map(int, line.split())) for line in lines[: len(cases)]], int(lines[len(cases)])
+
+    return run
+
+
+def test_every_ring_tile_has_a_gpu_shape(choose):
+    got, count = choose([(m, n, k, 256, True) for _, m, n, k in SHAPES])
+    for (tile, m, n, k), choice in zip(SHAPES, got):
+        assert choice == (*tile, 0), (m, n, k)
+    assert len({tile for tile, *_ in SHAPES}) == count
+
+
+def test_choices_by_hand(choose):
+    cases = [
+        # M = 4096, N = 17408, K = 5120: 1,248 persistent tiles, 4 + 0.75 + 0.25 * 224 / 256
+        # rounds of 52.5 us = 262 us; 22 x 109 = 2,398 tiles of 192 x 160, 9.37 + rounds of
+        # 38.7 us = 363 us.
+        (4096, 17408, 5120, 256, True),
+        # M = 128, N = K = 4096: 256 small-M tiles of 64 x 32, one round: 7.9 us; 256 ring
+        # tiles of 32 x 64: 8.9 us.
+        (128, 4096, 4096, 256, True),
+        # M = 1024, N = 5120, K = 17408: 256 tiles of 128 x 160, one round, 90.8 us; 92
+        # persistent tiles take 0.84 of a round of 155 us.
+        (1024, 5120, 17408, 256, True),
+        # M = 768, N = 17408, K = 5120: 234 persistent tiles, 0.98 of a round: 53 us; ring
+        # tiles take 2 rounds or more.
+        (768, 17408, 5120, 256, True),
+        # The same with an INT32 copy, which the persistent kernel does not write.
+        (768, 17408, 5120, 256, False),
+        # No CU count: the rules without a model.
+        (768, 17408, 5120, 0, True),
+    ]
+    got, _ = choose(cases)
+    assert got[0] == (0, 0, 1)
+    assert got[1] == (0, 0, 0)
+    assert got[2] == (128, 160, 0)
+    assert got[3] == (0, 0, 1)
+    assert got[4][0] > 0 and got[4][2] == 0
+    assert got[5] == (0, 0, 0)
