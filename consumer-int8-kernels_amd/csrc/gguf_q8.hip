@@ -15,8 +15,10 @@
 //
 // Kernels, all on v_mfma_f32_16x16x32_bf16 with the MFMA computing D[n][m] = Wq . x^T
 // (a lane holds 4 consecutive channels of one row and stores 8 bytes):
-//  * m <= 16, K <= 8192: the balanced-span kernel (the layout of the W8A16 GEMV).
-//  * m > 16: 256 x 128 or 128 x 128 tiles of eight waves with an LDS ring of three K
+//  * The ring kernel of gguf_ring.hip wherever its tiles are expected to finish first:
+//    m > 16 up to about a thousand rows, and m <= 16 with many channels (tile_plan.h).
+//  * Else m <= 16, K <= 8192: the balanced-span kernel (the layout of the W8A16 GEMV).
+//  * Else m > 16: 256 x 128 or 128 x 128 tiles of eight waves with an LDS ring of three K
 //    stages, codes dequantized once per tile and stage (gguf_q8_large_kernel).
 //  * Otherwise (x or the codes beyond a 2 GiB buffer range, or m <= 16 with K > 8192):
 //    a BM x 64 tile of four waves, each owning a 16-channel block and BM / 16 row blocks;
@@ -672,15 +674,21 @@ hipError_t launch_gguf_q8_packed_mm(const void* x, const int8_t* codes, const vo
   const auto* sp = static_cast<const uint16_t*>(scales);
   auto* op = static_cast<uint16_t*>(out);
   const unsigned tiles_n = unsigned((n + kBN - 1) / kBN);
+  const int cus = device_cu_count();
+  // The ring kernel where its tiles are expected to finish first (tile_plan.h), while x's
+  // and the codes' byte ranges fit a buffer's.
+  const bool buffers = (int64_t(m - 1) * xs + k) * 2 <= INT32_MAX && int64_t(n) * k <= INT32_MAX;
+  if (const int tile = buffers ? gguf_ring_tile(m, n, k, groups, cus) : -1;
+      tile >= 0 &&
+      tile_count(m, n, kGgufTiles[tile].bm, kGgufTiles[tile].bn) * groups <= INT32_MAX)
+    return launch_gguf_ring(tile, x, codes, scales, out, m, n, k, groups, xs, xg, stream);
   // m <= 16: the balanced-span kernel while each wave's K range holds its x fragments
   // in registers (K <= 16 ranges x 8 blocks x 64) and x's byte range fits a buffer.
-  const int cus = device_cu_count();
   const int range_len = (k / 64 + 15) / 16;
   // K > 8192 runs the span kernel in chunks of 8192 while a workgroup's partial sums of
   // all its channel blocks fit the LDS at once (span <= 8 blocks of 16).
   const int span_blocks = cus > 0 ? (span_channels(n, groups, cus) + 15) / 16 : 0;
-  if (m <= 16 && cus > 0 && (range_len <= 8 || span_blocks <= 8) &&
-      (int64_t(m - 1) * xs + k) * 2 <= INT32_MAX && int64_t(n) * k <= INT32_MAX) {
+  if (m <= 16 && cus > 0 && (range_len <= 8 || span_blocks <= 8) && buffers) {
     if (range_len <= 2)
       return run_span<GgufSpanConfig<2>>(x, codes, scales, out, m, n, k, groups, xs, xg, cus, stream);
     if (range_len <= 4)
@@ -693,13 +701,8 @@ hipError_t launch_gguf_q8_packed_mm(const void* x, const int8_t* codes, const vo
   // fit a buffer's), whichever takes fewer rounds of one tile per CU, a round of 256-row
   // tiles costing about 1.45 rounds of 128-row ones (measured on MI355X at K = 2048 ..
   // 5120; either beats the 64 x 64 tiles at every M from 64 up).
-  const int64_t tiles_n128 = (n + 127) / 128;
-  const int64_t tiles256 = (m + 255) / 256 * tiles_n128 * groups;
-  const int64_t tiles128 = (m + 127) / 128 * tiles_n128 * groups;
-  if (m > 16 && cus > 0 && (int64_t(m - 1) * xs + k) * 2 <= INT32_MAX &&
-      int64_t(n) * k <= INT32_MAX && tiles128 <= INT32_MAX) {
-    const int64_t rounds256 = (tiles256 + cus - 1) / cus, rounds128 = (tiles128 + cus - 1) / cus;
-    if (rounds256 * 29 <= rounds128 * 20)
+  if (m > 16 && cus > 0 && buffers && tile_count(m, n, 128, 128) * groups <= INT32_MAX) {
+    if (gguf_large_rows(m, n, groups, cus) == 256)
       return run_large<GgufLargeConfig<256>>(x, codes, scales, out, m, n, k, groups, xs, xg, stream);
     return run_large<GgufLargeConfig<128>>(x, codes, scales, out, m, n, k, groups, xs, xg, stream);
   }

@@ -99,6 +99,12 @@ hipError_t launch_gguf_q8_packed_mm(const void* x, const int8_t* codes, const vo
                                     void* out, int m, int n, int k, int groups, int64_t xs,
                                     int64_t xg, hipStream_t stream);
 
+// The same on tile kGgufTiles[tile] of tile_plan.h (gguf_ring.hip). Also requires x's byte
+// range within one group and n * k to be at most INT32_MAX.
+hipError_t launch_gguf_ring(int tile, const void* x, const int8_t* codes, const void* scales,
+                            void* out, int m, int n, int k, int groups, int64_t xs, int64_t xg,
+                            hipStream_t stream);
+
 hipError_t launch_channel_gemv(const void* x, const int8_t* w, const void* scale, void* out,
                                int m, int n, int k, hipStream_t stream);
 

@@ -230,4 +230,44 @@ inline GemmChoice gemm_choice(int m, int n, int k, int cus, bool persistent_ok) 
   return choice;
 }
 
+// Tiles of the GGUF ring kernel (gguf_ring.hip) with the time of a round, as kRingTiles:
+// fitted to 162 shapes measured on MI355X (M = 1..3000; (N, K, groups) = (4096, 4096, 1),
+// (1925, 2176, 1), (2808, 1792, 1), (1085, 1664, 4), (8192, 8192, 1), (3555, 3584, 1), (1024,
+// 1024, 1), (5120, 2048, 2), (6000, 6016, 1)), rms error 5-8%.
+constexpr RingTile kGgufTiles[] = {
+    {16, 16, 1.9, 1.02}, {16, 32, 3.0, 1.25}, {32, 32, 3.5, 1.48},
+    {64, 32, 4.9, 1.79}, {64, 64, 4.9, 3.15}, {96, 64, 6.1, 3.84},
+    {128, 64, 6.6, 4.76}, {128, 96, 8.1, 6.50}, {128, 128, 10.0, 7.99}};
+constexpr int kGgufTileCount = sizeof(kGgufTiles) / sizeof(kGgufTiles[0]);
+
+// The ring tile for gguf_q8_packed_mm, or -1 where gguf_q8.hip's kernels are expected to be
+// faster: its span kernel up to M = 16 (time in channels per CU: 0.95 us per 16 channels
+// and 1024 of K at M = 1, 1.4 at M = 16, past 3.2 us), its 256- or 128-row tiles beyond
+// (large_rows, of which it takes the one with fewer rounds). With the measured times the
+// choice is within 1% of the best kernel in the mean.
+inline int gguf_large_rows(int m, int n, int groups, int cus) {
+  const int64_t tiles256 = tile_count(m, n, 256, 128) * groups;
+  const int64_t tiles128 = tile_count(m, n, 128, 128) * groups;
+  return (tiles256 + cus - 1) / cus * 29 <= (tiles128 + cus - 1) / cus * 20 ? 256 : 128;
+}
+inline int gguf_ring_tile(int m, int n, int k, int groups, int cus) {
+  if (cus <= 0) return -1;
+  double best;
+  if (m <= 16) {
+    const double channels = double((int64_t(n) * groups + cus - 1) / cus);
+    best = 3.2 + channels / 16 * k / 1024 * (0.95 + 0.027 * m);
+  } else {
+    const int rows = gguf_large_rows(m, n, groups, cus);
+    best = tiled_time(tile_count(m, n, rows, 128) * groups, cus, rows == 256 ? 8.6 : 4.4,
+                      rows == 256 ? 14.2 : 10.7, k);
+  }
+  int tile = -1;
+  for (int i = 0; i < kGgufTileCount; ++i) {
+    const RingTile& t = kGgufTiles[i];
+    const double time = tiled_time(tile_count(m, n, t.bm, t.bn) * groups, cus, t.fixed, t.per_k, k);
+    if (time < best) best = time, tile = i;
+  }
+  return tile;
+}
+
 }  // namespace ci8
