@@ -1444,15 +1444,22 @@ hipError_t launch_channel_gemm(const int8_t* a, const void* w, WeightCode code,
 hipError_t launch_grouped_summed_gemm(const int8_t* a, const int8_t* w, const float* sa,
                                       const void* sw, void* out, int groups, int m, int n,
                                       int k, hipStream_t stream) {
-  if (m <= 32) return run_grouped<Small>(a, w, sa, sw, out, groups, m, n, k, stream);
   // The two-waves-per-SIMD kernel copies the row scales into LDS four rows (16 bytes) at a
   // time at byte offset 4 (g m + row) of a buffer of 4 groups m bytes: that needs m % 4 == 0
   // and a 16-byte aligned sa (so no copy straddles a group boundary, is misaligned or runs
   // past the end of sa), and every offset below the 2^31 out-of-range marker.
-  if (m >= 1024 && n % 4 == 0 && reinterpret_cast<uintptr_t>(sw) % 8 == 0 &&
+  const bool persistent_ok =
+      m >= 1024 && n % 4 == 0 && reinterpret_cast<uintptr_t>(sw) % 8 == 0 &&
       groups <= grouped_pp_max_groups() && m % 4 == 0 &&
       reinterpret_cast<uintptr_t>(sa) % 16 == 0 &&
-      int64_t(groups) * m * 4 < (int64_t(1) << 31))
+      int64_t(groups) * m * 4 < (int64_t(1) << 31);
+  // The ring kernel (grouped_ring.hip) unless that kernel is expected to be faster; past its
+  // LDS for row scales, the 32 x 32-MFMA kernel above.
+  if (const int tile = grouped_ring_tile(m, n, k, groups, device_cu_count(), persistent_ok);
+      tile >= 0)
+    return launch_grouped_ring_gemm(tile, a, w, sa, sw, out, groups, m, n, k, stream);
+  if (m <= 32) return run_grouped<Small>(a, w, sa, sw, out, groups, m, n, k, stream);
+  if (persistent_ok)
     return launch_grouped_pp_gemm(a, w, sa, sw, out, groups, m, n, k, stream);
   return run_grouped<Medium>(a, w, sa, sw, out, groups, m, n, k, stream);
 }

@@ -70,6 +70,12 @@ hipError_t launch_grouped_pp_gemm(const int8_t* a, const int8_t* w, const float*
                                   const void* sw, void* out, int groups, int m, int n, int k,
                                   hipStream_t stream);
 
+// The same on tile kGroupedTiles[tile] of tile_plan.h (grouped_ring.hip); identical bits.
+// Requires a and w 16-byte aligned and groups * bm * 4 <= kGroupedScaleBytes.
+hipError_t launch_grouped_ring_gemm(int tile, const int8_t* a, const int8_t* w, const float* sa,
+                                    const void* sw, void* out, int groups, int m, int n, int k,
+                                    hipStream_t stream);
+
 // x BF16 [m, 2k] = [gate | up] -> out BF16 [m, k] = bf16(silu(gate) * up).
 hipError_t launch_silu_mul(const void* x, void* out, int m, int k, hipStream_t stream);
 // The same activations quantized per row like launch_quantize_rows, never written out.

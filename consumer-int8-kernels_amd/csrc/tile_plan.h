@@ -270,4 +270,37 @@ inline int gguf_ring_tile(int m, int n, int k, int groups, int cus) {
   return tile;
 }
 
+// Tiles of the grouped ring kernel (grouped_ring.hip) with the time of a round, `per_k` per
+// 1024 of the K of all groups: fitted to 105 shapes measured on MI355X (M = 17..4096; (N,
+// groups, K) = (4096, 4, 4096), (4616, 1, 4096), (2456, 3, 4096), (1496, 2, 4096), (8192, 2,
+// 4096), (1024, 1, 4096), (3000, 3, 1056)), rms error 5-7%.
+constexpr RingTile kGroupedTiles[] = {
+    {32, 64, 3.1, 1.47},  {64, 64, 4.2, 1.89},   {96, 64, 4.6, 2.43},  {64, 96, 5.3, 2.44},
+    {64, 128, 5.8, 2.74}, {96, 128, 6.4, 3.87},  {128, 96, 6.7, 3.89}, {128, 128, 7.1, 4.47},
+    {160, 128, 8.4, 5.34}, {192, 128, 8.3, 6.01}};
+constexpr int kGroupedTileCount = sizeof(kGroupedTiles) / sizeof(kGroupedTiles[0]);
+// LDS kept for a tile's row scales of all groups, four bytes a row and group.
+constexpr int kGroupedScaleBytes = 16 * 1024;
+
+// The grouped ring tile, or -1 where the two-waves-per-SIMD kernel's 256 x 128 tiles
+// (persistent_ok: it can run this call; 6.6 us per 1024 of K and round, past 7.8) are
+// expected to be faster or the row scales of a tile do not fit. It always beats the 32 x
+// 32-MFMA kernel (by 1.3 to 4 times at all 105 shapes). The choice is within 1% of the best
+// kernel in the mean.
+inline int grouped_ring_tile(int m, int n, int k, int groups, int cus, bool persistent_ok) {
+  if (cus <= 0) return -1;
+  auto time = [&](int bm, int bn, double fixed, double per_k) {
+    return tiled_time(tile_count(m, n, bm, bn), cus, fixed, per_k * groups, k);
+  };
+  int tile = -1;
+  double best = persistent_ok ? time(256, 128, 7.8, 6.6) : 0.0;
+  for (int i = 0; i < kGroupedTileCount; ++i) {
+    const RingTile& t = kGroupedTiles[i];
+    if (int64_t(groups) * t.bm * 4 > kGroupedScaleBytes) continue;
+    const double us = time(t.bm, t.bn, t.fixed, t.per_k);
+    if ((tile < 0 && !persistent_ok) || us < best) best = us, tile = i;
+  }
+  return tile;
+}
+
 }  // namespace ci8
