@@ -30,7 +30,7 @@ ROCM = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
 HIPCC = str(ROCM / "bin" / "hipcc")
 ARCH = "gfx950"
 
-HIP_SOURCES = ["quantize.hip", "gemm.hip", "gemm_small.hip", "gemm_ring.hip", "gemm_pp.hip", "gemv.hip", "silu.hip",
+HIP_SOURCES = ["quantize.hip", "gemm.hip", "gemm_small.hip", "gemm_ring.hip", "gemm_pp.hip", "gemv.hip", "gemv_stream.hip", "silu.hip",
                "allspark.hip", "q8block.hip", "gguf_q8.hip", "gguf_ring.hip",
                "gemm_grouped.hip", "grouped_ring.hip", "noalloc.hip", "gemm_bytes.hip"]
 HOST_SOURCES = ["abi.cpp"]

@@ -1011,9 +1011,14 @@ hipError_t run_quad(const void* x, const int8_t* w, const void* scale, void* out
 
 hipError_t launch_channel_gemv(const void* x, const int8_t* w, const void* scale, void* out,
                                int m, int n, int k, hipStream_t stream) {
+  const int cus = device_cu_count();
+  // The stream kernel (gemv_stream.hip) where it is the faster one (tile_plan.h), for an x
+  // that its 16-byte copies can read.
+  if (const int copies = gemv_stream_copies(m, n, k, cus);
+      copies > 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0)
+    return launch_stream_gemv(copies, x, w, scale, out, m, n, k, stream);
   // K <= 8192 and m >= 2: the balanced-span kernel (measured on MI355X at K = 5120, N =
   // 17408: 20.2 - 22.9 us over m = 2 .. 16, against 20.4 - 30.9 us for the kernels below).
-  const int cus = device_cu_count();
   // 2 <= m <= 4 with 4096 <= K <= 8192, and 5 <= m <= 8 with 5120 < K <= 8192: the
   // interleaved quad-block kernel (measured at K = 5120, N = 17408: 16.3 / 17.1 us at
   // m = 2 / 4 against 19.6 / 19.9 us for the span kernel; at N = K = 8192, m = 5 .. 8:

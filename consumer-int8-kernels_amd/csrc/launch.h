@@ -111,6 +111,11 @@ hipError_t launch_gguf_ring(int tile, const void* x, const int8_t* codes, const 
                             void* out, int m, int n, int k, int groups, int64_t xs, int64_t xg,
                             hipStream_t stream);
 
+// channel_gemv with 8 * copies channels per workgroup (gemv_stream.hip; 1 <= copies <=
+// kStreamMaxCopies). Requires x and w 16-byte aligned and k % 16 == 0.
+hipError_t launch_stream_gemv(int copies, const void* x, const int8_t* w, const void* scale,
+                              void* out, int m, int n, int k, hipStream_t stream);
+
 hipError_t launch_channel_gemv(const void* x, const int8_t* w, const void* scale, void* out,
                                int m, int n, int k, hipStream_t stream);
 

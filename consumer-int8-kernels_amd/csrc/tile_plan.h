@@ -303,4 +303,26 @@ inline int grouped_ring_tile(int m, int n, int k, int groups, int cus, bool pers
   return tile;
 }
 
+// channel_gemv: 8-channel copies per stage of the stream kernel (gemv_stream.hip) that fill
+// the CUs in as few rounds of one tile each as its widest tile allows, or 0 where gemv.hip's
+// kernels are faster. Measured on MI355X at 20 shapes and M = 1..16 (stream against those, us):
+//   K > 8192: everywhere (5120 x 17408: 18.9-24.4 against 23.1-30.9; 3376 x 8704, M = 1: 7.6
+//     against 7.9; 2560 x 10240, M = 8: 8.5 against 17.0);
+//   M >= 5, up to 20 channels a CU: the span and quad kernels pad to 16 channels and one
+//     round's latency (4096 x 4096: 6.2-6.6 against 7.5-8.3; 5120 x 5120: 8.2-9.4 against
+//     8.5-10.9);
+//   M >= 9, K >= 5120, up to 40 channels a CU: 7168 x 5120 9.8-9.9 against 9.8-11.4, 8192 x
+//     8192 15.8-16.7 against 17.4-19.3. Beyond, the span kernel is level or faster (12000 x
+//     6000, M = 9: 15.9 against 16.3; 28672 x 8192: 48.5 against 51.0), and so are the row
+//     and quad kernels at M <= 4 (17408 x 5120, M = 2: 15.6 against 18.7).
+constexpr int kStreamMaxCopies = 9;
+inline int gemv_stream_copies(int m, int n, int k, int cus) {
+  if (cus <= 0) return 0;
+  const int64_t channels = (int64_t(n) + cus - 1) / cus;
+  if (!(k > 8192 || (m >= 5 && channels <= 20) || (m >= 9 && k >= 5120 && channels <= 40)))
+    return 0;
+  const int64_t rounds = (channels + 8 * kStreamMaxCopies - 1) / (8 * kStreamMaxCopies);
+  return int(((int64_t(n) + cus * rounds - 1) / (cus * rounds) + 7) / 8);
+}
+
 }  // namespace ci8
