@@ -1227,8 +1227,8 @@ using Pipe224 = K128Config<256, 224, 2, 2, 8>;        // 4 waves, 128x112 per wa
 using WLds224 = WLdsConfig<224, 8, true>;             // 4 waves, 64x224 per wave
 using WLds256 = WLdsConfig<256, 8, false>;            // 4 waves, 64x256 per wave
 
-// wide_tiles_pay and pp_beats_wide_tiles (tile_plan.h) choose between the 224-wide,
-// 256-wide and persistent kernels.
+// wide_tiles_pay and gemm_choice (tile_plan.h) choose between the 224-wide, 256-wide and
+// persistent kernels.
 static_assert(WLds256::BN == kPlanWideBN && WLds224::BN == kPlanBN, "tile_plan.h widths");
 
 template <WeightCode kCode, bool kWorkspace>
@@ -1258,14 +1258,10 @@ hipError_t dispatch(const int8_t* a, const void* w, const float* sa, const void*
   if (choice == 0)
     choice = m < 1024 || medium_tiles_pay(m, n, cus) ? 1 : (wide_tiles_pay(m, n, cus) ? 3 : 4);
   // Without the INT32 copy, M >= 1024: the persistent two-waves-per-SIMD kernel
-  // (gemm_pp.hip) for either weight code (its epilogue reads the channel scales 8 bytes
-  // at a time) in place of the 224-wide one, and also in place of the 256-wide one
-  // unless that needs far fewer rounds: per MFMA it is about 1.2x as fast (configs[3],
-  // M = 16384, K = 17408, N = 5120: 5 rounds of 224-wide tiles and one of 160-wide beat 5
-  // rounds of 256-wide; M = N = 4096: 2 rounds lose to 1).
+  // (gemm_pp.hip) for either weight code (its epilogue reads the channel scales 8 bytes at a
+  // time) in place of the 224-wide one: per MFMA it is about 1.2x as fast.
   if constexpr (!kWorkspace) {
-    if (schedule == 0 && m >= 1024 && choice != 1 && persistent_ok &&
-        (choice == 4 || pp_beats_wide_tiles(m, n, cus)))
+    if (schedule == 0 && m >= 1024 && choice == 4 && persistent_ok)
       return launch_pp_gemm(a, w, kCode, sa, sw, out, m, n, k, stream);
   }
   switch (choice) {

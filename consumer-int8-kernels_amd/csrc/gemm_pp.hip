@@ -8,20 +8,22 @@
 // per four bytes after each W fragment read.
 //
 // Persistent: one workgroup of eight waves per CU walks the 256 (m) x 224 (n) output
-// tiles b, b + grid, ... (grid = CU count). Where the 224-wide tiles would leave the last
-// round partly empty and 160-wide tiles fill it, the columns are split between two
-// launches (pp_plan below): whole rounds of 224-wide tiles, then 160-wide tiles over the
-// rest (configs[3], M = 16384, N = 5120: 5 rounds over 4480 columns, then one round of
-// 256 x 160 tiles over 640, in place of 5.75 rounds of 224-wide tiles). The 160-wide
-// kernel is the same source with 5 n blocks per wave, 5 W copies per W wave and a copy
-// after every second fragment read (gemm_pp_kernel.h); the numbers below are the 224-wide
-// kernel's.
+// tiles b, b + grid, ... (grid = CU count). Tiles of 192, 160 or 128 columns take the whole
+// launch where they fill its rounds better (pp_width, tile_plan.h; M = 2048, N = K = 4096:
+// 256 tiles of 128 in place of 152 of 224, 39.1 -> 34.3 us; M = 4096, N = K = 8192, 192 wide:
+// 237.8 -> 216.8). Where the 224-wide tiles stay and would leave the last round partly empty,
+// the columns may be split between two launches (pp_plan): whole rounds of 224-wide tiles,
+// then 160-wide tiles over the rest (M = 16384, N = 5120, K = 17408: 5 rounds over 4480
+// columns, then one round of 256 x 160 tiles over 640, in place of 5.75 rounds of 224-wide
+// tiles). The narrower kernels are the same source with fewer n blocks and W copies per wave
+// (160: 5 of each, a copy after every second fragment read; gemm_pp_kernel.h); the numbers
+// below are the 224-wide kernel's.
 //
 // The copy stream runs on across tiles: the K
 // stages g = r * ns + t of the whole launch (tile r, stage t) use ring slots g % 2 (A)
 // and g % 3 (W), and a tile's last stages copy the next tile's first stages just as they
 // copy their own, so the tile switch issues no copies and the address unit is free for
-// the epilogue's stores (measured on MI355X at configs[2]: 105 K against 108 K cycles
+// the epilogue's stores (measured on MI355X, M = 4096, N = 17408, K = 5120: 105 K against 108 K cycles
 // per tile, 255.6-257.4 against 259.6-261.0 us, identical outputs). The epilogue runs
 // through the A slot of the tile's last stage, which the next tile's first copies do not
 // use. The tile's row and channel scales are copied into LDS at the tile start and read
@@ -110,6 +112,17 @@ hipError_t launch_pp_gemm(const int8_t* a, const void* w, WeightCode code, const
     return exact ? go(kernel_constant<pp_gemm_kernel<true, kU, 0, kBN>>{})
                  : go(kernel_constant<pp_gemm_kernel<false, kU, 0, kBN>>{});
   };
+  // One launch of narrower tiles where they fill the rounds better (pp_width, tile_plan.h).
+  switch (pp_width(m, n, k, cus).bn) {
+    case 192:
+      return launch(std::integral_constant<int, 192>{}, 0, n);
+    case PPConfigNarrow::BN:
+      return launch(std::integral_constant<int, PPConfigNarrow::BN>{}, 0, n);
+    case 128:
+      return launch(std::integral_constant<int, 128>{}, 0, n);
+    default:
+      break;
+  }
   const PPPlan plan = pp_plan(m, n, cus);
   if (plan.n_head == 0) return launch(std::integral_constant<int, PPConfig::BN>{}, 0, n);
   if (const hipError_t e = launch(std::integral_constant<int, PPConfig::BN>{}, 0, plan.n_head);

@@ -12,8 +12,8 @@ namespace {
 
 constexpr int kXcds = 8;
 
-// Tiles of 256 (m) x kBN (n), kBN = 224 (the default) or 160 (the narrow tiles that let
-// a launch end in whole rounds; see launch_pp_gemm). Group g = wave / 4 owns WN = kBN / 2
+// Tiles of 256 (m) x kBN (n), kBN = 224 (the default) or 192, 160 or 128 (narrower tiles
+// that let a launch end in whole rounds; see launch_pp_gemm). Group g = wave / 4 owns WN = kBN / 2
 // columns of the tile.
 template <int kBN>
 struct PPConfigT {

@@ -11,12 +11,12 @@ namespace ci8 {
 constexpr int kPlanBM = 256, kPlanBN = 224, kPlanNarrowBN = 160, kPlanWideBN = 256;
 
 // Time of a round of 160-wide tiles, in units where a round of 224-wide tiles takes 224
-// (measured on MI355X at configs[3], M = 16384, K = 17408: 5 rounds of 224-wide tiles
+// (measured on MI355X, M = 16384, K = 17408: 5 rounds of 224-wide tiles
 // over N = 4480 took 966-978 us, and the split launch over N = 5120 1114-1129 us, so the
 // 160-wide round and the second launch took ~0.8 of a 224-wide round).
 //
 // The split gains less than its rounds suggest: the chip runs at its power limit, so a
-// partly filled last round runs faster per tile than a full one. At configs[3] the single
+// partly filled last round runs faster per tile than a full one. There the single
 // launch's sixth round (192 of 256 CUs busy, 672 columns for 640) took ~161 us against
 // ~195 us for a full round, and the split launch measured 1114-1129 against 1131-1145 us
 // (same process, alternating, identical outputs; at K = 5120, 326.5-327.7 against
@@ -24,7 +24,8 @@ constexpr int kPlanBM = 256, kPlanBN = 224, kPlanNarrowBN = 160, kPlanWideBN = 2
 // compute.
 constexpr int64_t kNarrowRoundCost = 180;
 
-// Column plan of the two-waves-per-SIMD GEMM (gemm_pp.hip) at m x n on `cus` CUs: 224-wide
+// Column plan of the two-waves-per-SIMD GEMM (gemm_pp.hip) at m x n on `cus` CUs where
+// pp_width (below) picks its 224-wide tiles: 224-wide
 // tiles over the first n_head columns and 160-wide tiles over the rest (n_head = 0: one
 // launch of 224-wide tiles over all n). `cost` is the planned rounds' time in units where a
 // round of 224-wide tiles takes 224.
@@ -153,7 +154,7 @@ inline bool medium_tiles_pay(int m, int n, int cus) {
   return 2 * tiles224 < cus && tiles128 <= cus;
 }
 
-// Tiles of the ring kernel (gemm_mid.hip), each with the time of a round of them (one tile
+// Tiles of the ring kernel (gemm_ring.hip), each with the time of a round of them (one tile
 // on every CU): `fixed` + `per_k` * K / 1024 us. Fitted to 162 shapes measured on MI355X
 // (M = 17..3000 with (N, K) = 4096 x 4096, 17408 x 5120, 5120 x 17408, 7168 x 5120, 5120 x
 // 8704, 2048 x 8192, 1000 x 1024, 3000 x 2048 and 12000 x 3072; three rotated weight
@@ -172,8 +173,8 @@ constexpr RingTile kRingTiles[] = {
 constexpr int kRingTileCount = sizeof(kRingTiles) / sizeof(kRingTiles[0]);
 
 // Time (us) of one launch of a tiled GEMM that runs its tiles in rounds of one per CU: a
-// round of the other kernels' tiles by the same measurements (the persistent kernel's 256 x
-// 224 tiles; 256-wide tiles of the one-wave-per-SIMD kernel; the small-M kernel below). A
+// round of the other kernels' tiles by the same measurements (the persistent kernel's tiles;
+// 256-wide tiles of the one-wave-per-SIMD kernel; the small-M kernel below). A
 // last round that is not full takes three quarters of a round plus its share of the rest
 // (fewer CUs share the caches and the power; the best single share over all tiles).
 constexpr double kLaunchTime = 1.5;
@@ -188,8 +189,38 @@ inline int64_t tile_count(int m, int n, int bm, int bn) {
 inline double ring_time(const RingTile& t, int m, int n, int k, int cus) {
   return tiled_time(tile_count(m, n, t.bm, t.bn), cus, t.fixed, t.per_k, k);
 }
+// Widths of the persistent kernel's tiles (256 rows each) with the time of a round, fitted to
+// 122 shapes measured on MI355X (M = 320..16384; (N, K) = 17408 x 5120, 5120 x 17408, 7168 x
+// 5120, 5120 x 8704, 4096 x 4096, 12000 x 3072, 8192 x 8192, 2560 x 10240, 8448 x 128, 4096 x
+// 256, 12000 x 512, 8192 x 1024, 5120 x 2048, 20000 x 1024, 6144 x 8192; rms error 6-7%). A
+// narrower tile costs more per column (more operand bytes per MFMA) and pays where it fills
+// the rounds better: M = 2048, N = 5120, K = 17408 is 184 tiles of 224 or 256 of 160, one
+// round each, 157.8 against 151.8 us; M = 2560, N = 12000, K = 3072 is 540 of 224 (95.0 us;
+// 101.7 split) or 760 of 160, 85.8. With these times the choice of kernel and width is 0.5%
+// off the best in the mean; with 224-wide tiles alone it was 3.7%.
+struct PPWidth {
+  int bn;
+  double fixed, per_k;
+};
+constexpr PPWidth kPPWidths[] = {
+    {kPlanBN, 9.1, 8.71}, {192, 6.9, 7.90}, {kPlanNarrowBN, 6.3, 7.23}, {128, 4.5, 6.77}};
+inline double persistent_time(const PPWidth& w, int m, int n, int k, int cus) {
+  return tiled_time(tile_count(m, n, kPlanBM, w.bn), cus, w.fixed, w.per_k, k);
+}
+// The width of a whole launch. 224 (which pp_plan may still split) unless another one is
+// expected to save 1%; launch_pp_gemm runs it. cus <= 0: 224.
+inline const PPWidth& pp_width(int m, int n, int k, int cus) {
+  const PPWidth* best = kPPWidths;
+  if (cus <= 0) return *best;
+  double time = 0.99 * persistent_time(*best, m, n, k, cus);
+  for (const PPWidth& w : kPPWidths) {
+    const double t = persistent_time(w, m, n, k, cus);
+    if (t < time) time = t, best = &w;
+  }
+  return *best;
+}
 inline double persistent_time(int m, int n, int k, int cus) {
-  return tiled_time(tile_count(m, n, kPlanBM, kPlanBN), cus, 9.7, 8.56, k);
+  return persistent_time(pp_width(m, n, k, cus), m, n, k, cus);
 }
 inline double wide_time(int m, int n, int bn, int k, int cus) {
   return tiled_time(tile_count(m, n, kPlanBM, bn), cus, 9.7, 13.8 * bn / kPlanWideBN, k);
@@ -205,7 +236,7 @@ inline double small_time(int m, int n, int k, int cus) {
 // kernel is taken where its best tile is expected to beat the kernel that those rules take
 // (the small-M kernel up to kSmallMaxM, the persistent or the one-wave-per-SIMD kernel from
 // M = 1024 on) and the persistent kernel. The persistent kernel is also taken below M =
-// 1024 where its 256 x 224 tiles fill most of a round. persistent_ok: it can run this call.
+// 1024 where its tiles fill most of a round. persistent_ok: it can run this call.
 struct GemmChoice {
   int ring;
   bool persistent;
@@ -221,9 +252,16 @@ inline GemmChoice gemm_choice(int m, int n, int k, int cus, bool persistent_ok) 
   if (m <= kSmallMaxM && small_time(m, n, k, cus) <= best) return {-1, false};
   if (m <= kSmallOnlyMaxM) return choice;
   if (persistent_ok) {
-    if (m >= 1024 && !pp_beats_wide_tiles(m, n, cus))
-      return wide_time(m, n, kPlanWideBN, k, cus) <= best ? GemmChoice{-1, false} : choice;
-    return persistent_time(m, n, k, cus) <= best ? GemmChoice{-1, true} : choice;
+    // Where 224-wide persistent tiles lose to 256-wide ones on rounds, another width or the
+    // ring kernel has to be expected 5% below those: M = 4096, N = K = 8192 (two full rounds
+    // of 256, 2.69 of 192) 237.8 -> 216.8 us; M = 2048, N = K = 8192 (one round of 256, two of
+    // 128, 2% below by the model) measured 118.8 against 124.9, M = 3072, N = 5120, K = 8192
+    // (240 of 256, ring 2% below) 112.6 against 119.1.
+    const double time = persistent_time(m, n, k, cus);
+    const double wide = 0.95 * wide_time(m, n, kPlanWideBN, k, cus);
+    if (m >= 1024 && !pp_beats_wide_tiles(m, n, cus) && wide <= time)
+      return wide <= best ? GemmChoice{-1, false} : choice;
+    return time <= best ? GemmChoice{-1, true} : choice;
   }
   const int wide = wide_tiles_pay(m, n, cus) ? kPlanWideBN : kPlanBN;
   if (m >= 1024 && wide_time(m, n, wide, k, cus) <= best) return {-1, false};

@@ -20,9 +20,9 @@ SHAPES = [
     ((32, 96), 13, 16756, 160), ((64, 48), 334, 1476, 1696), ((64, 64), 353, 2452, 1120),
     ((64, 64), 37, 13132, 1472), ((64, 80), 938, 1188, 1920), ((64, 96), 375, 4028, 1984),
     ((64, 128), 669, 2780, 1888), ((96, 96), 1234, 1560, 1856), ((128, 80), 501, 4104, 1696),
-    ((96, 128), 473, 5228, 928), ((128, 128), 328, 10808, 1728), ((128, 128), 293, 8472, 32),
-    ((128, 160), 641, 5704, 32), ((128, 160), 1157, 3384, 416), ((160, 160), 1385, 4312, 1184),
-    ((192, 128), 563, 10156, 288), ((192, 160), 849, 7592, 544),
+    ((96, 128), 473, 5228, 928), ((128, 128), 328, 10808, 1728), ((128, 128), 297, 8468, 416),
+    ((128, 160), 1061, 3724, 1056), ((128, 160), 293, 10948, 800), ((160, 160), 401, 10260, 2080),
+    ((192, 128), 521, 8196, 1184), ((192, 160), 521, 10948, 800),
 ]
 
 

@@ -9,6 +9,7 @@ import subprocess
 import pytest
 
 from tests.conftest import PKG
+from tests.test_gpu_pp_width import SHAPES as PP_SHAPES
 from tests.test_gpu_ring import SHAPES
 
 PROGRAM = r"""
@@ -20,8 +21,10 @@ int main(int argc, char** argv) {
   for (int i = 1; i + 4 < argc; i += 5) {
     const GemmChoice c = gemm_choice(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]),
                                      atoi(argv[i + 3]), atoi(argv[i + 4]) != 0);
+    const int width = pp_width(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]),
+                               atoi(argv[i + 3])).bn;
     std::printf("%d %d %d\n", c.ring < 0 ? 0 : kRingTiles[c.ring].bm,
-                c.ring < 0 ? 0 : kRingTiles[c.ring].bn, int(c.persistent));
+                c.ring < 0 ? 0 : kRingTiles[c.ring].bn, c.persistent ? width : 0);
   }
   std::printf("%d\n", kRingTileCount);
   return 0;
@@ -55,17 +58,23 @@ def test_every_ring_tile_has_a_gpu_shape(choose):
     assert len({tile for tile, *_ in SHAPES}) == count
 
 
+def test_persistent_widths_have_gpu_shapes(choose):
+    got, _ = choose([(m, n, k, 256, True) for _, m, n, k in PP_SHAPES])
+    assert got == [(0, 0, width) for width, *_ in PP_SHAPES]
+    assert {width for width, *_ in PP_SHAPES} == {224, 192, 160, 128}
+
+
 def test_choices_by_hand(choose):
     cases = [
         # M = 4096, N = 17408, K = 5120: 1,248 persistent tiles, 4 + 0.75 + 0.25 * 224 / 256
-        # rounds of 52.5 us = 262 us; 22 x 109 = 2,398 tiles of 192 x 160, 9.37 + rounds of
+        # rounds of 52.7 us = 263 us; 22 x 109 = 2,398 tiles of 192 x 160, 9.37 + rounds of
         # 38.7 us = 363 us.
         (4096, 17408, 5120, 256, True),
         # M = 128, N = K = 4096: 256 small-M tiles of 64 x 32, one round: 7.9 us; 256 ring
         # tiles of 32 x 64: 8.9 us.
         (128, 4096, 4096, 256, True),
         # M = 1024, N = 5120, K = 17408: 256 tiles of 128 x 160, one round, 90.8 us; 92
-        # persistent tiles take 0.84 of a round of 155 us.
+        # persistent tiles of 224 take 0.84 of a round of 157 us, 160 of 128 0.91 of 120 us.
         (1024, 5120, 17408, 256, True),
         # M = 768, N = 17408, K = 5120: 234 persistent tiles, 0.98 of a round: 53 us; ring
         # tiles take 2 rounds or more.
@@ -74,11 +83,15 @@ def test_choices_by_hand(choose):
         (768, 17408, 5120, 256, False),
         # No CU count: the rules without a model.
         (768, 17408, 5120, 0, True),
+        # M = 2048, N = 5120, K = 17408: 256 tiles of 256 x 160, one round, 129 us; 184 of 224
+        # 0.93 of a round of 157 us, 216 of 192 0.96 of one of 141 us.
+        (2048, 5120, 17408, 256, True),
     ]
     got, _ = choose(cases)
-    assert got[0] == (0, 0, 1)
+    assert got[0] == (0, 0, 224)
     assert got[1] == (0, 0, 0)
     assert got[2] == (128, 160, 0)
-    assert got[3] == (0, 0, 1)
+    assert got[3] == (0, 0, 224)
     assert got[4][0] > 0 and got[4][2] == 0
     assert got[5] == (0, 0, 0)
+    assert got[6] == (0, 0, 160)
