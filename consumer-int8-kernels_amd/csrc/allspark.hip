@@ -13,9 +13,11 @@
 // the lanes of a wave take consecutive tiles, so together they read 4 KiB of one packed
 // row), rebuilds the four output rows' 16-byte pieces with byte selects and a XOR of
 // 0x80 per byte, and stores them; consecutive lanes write consecutive 16-byte pieces of
-// each output row (nontemporal stores: the restored layer is not read back by this
-// kernel). Rows at or beyond n (the last group when n % 32 == 16) are neither stored nor
-// their bytes used. Pure data movement: HBM-bound at 2 bytes per weight.
+// each output row (stored through the caches while the layer fits the MALL, stream_policy
+// in ci8_device.h: the GEMM that follows reads it; M = 256, N = 7168, K = 5120 with quantizer
+// and GEMM 40.6 -> 36.7 us, N = 17408 80.2 -> 75.4, though the kernel alone takes 14.2 for
+// 13.6 and 38.5 for 30.9). Rows at or beyond n (the last group when n % 32 == 16) are
+// neither stored nor their bytes used. Pure data movement: HBM-bound at 2 bytes per weight.
 #include "ci8_device.h"
 #include "launch.h"
 
@@ -31,8 +33,8 @@ __device__ __forceinline__ u32x4 restore_piece(uint32_t a, uint32_t b, uint32_t 
 }
 
 // blockIdx.y = packed row p, lanes over tiles. kVec: packed is 16-byte aligned (else
-// 4-byte words).
-template <bool kVec>
+// 4-byte words). kPolicy: stores only; the loads are plain.
+template <bool kVec, StreamPolicy kPolicy>
 __global__ void __launch_bounds__(256) unpack_allspark_kernel(
     const uint8_t* __restrict__ packed, const uint16_t* __restrict__ packed_scales,
     int8_t* __restrict__ weight, uint16_t* __restrict__ scales, int n, int k) {
@@ -58,7 +60,7 @@ __global__ void __launch_bounds__(256) unpack_allspark_kernel(
   for (int q = 0; q < 4; ++q) {
     const int row = first + 8 * q;
     if (row < n)
-      __builtin_nontemporal_store(
+      stream_store<kPolicy>(
           restore_piece(chunk[0][q], chunk[1][q], chunk[2][q], chunk[3][q]),
           reinterpret_cast<u32x4*>(weight + int64_t(row) * k + int64_t(tile) * 16));
   }
@@ -80,10 +82,15 @@ hipError_t launch_unpack_allspark(const uint8_t* packed, const void* packed_scal
   const dim3 grid((k / 16 + 255) / 256, packed_rows);
   const auto* ps = static_cast<const uint16_t*>(packed_scales);
   auto* s = static_cast<uint16_t*>(scales);
-  if (reinterpret_cast<uintptr_t>(packed) % 16 == 0)
-    unpack_allspark_kernel<true><<<grid, 256, 0, stream>>>(packed, ps, weight, s, n, k);
+  const bool vec = reinterpret_cast<uintptr_t>(packed) % 16 == 0;
+  const bool nt = stream_policy(0, int64_t(n) * k) == kNtLoadsAndStores;
+  auto go = [&](auto kernel) { kernel<<<grid, 256, 0, stream>>>(packed, ps, weight, s, n, k); };
+  if (vec)
+    go(nt ? unpack_allspark_kernel<true, kNtLoadsAndStores>
+          : unpack_allspark_kernel<true, kCached>);
   else
-    unpack_allspark_kernel<false><<<grid, 256, 0, stream>>>(packed, ps, weight, s, n, k);
+    go(nt ? unpack_allspark_kernel<false, kNtLoadsAndStores>
+          : unpack_allspark_kernel<false, kCached>);
   return hipGetLastError();
 }
 

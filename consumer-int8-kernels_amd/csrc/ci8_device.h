@@ -84,12 +84,36 @@ __device__ __forceinline__ u32x2 codes8(const u32x4& packed, float scale, float 
   return out;
 }
 
-// Inputs larger than MI355X's 256 MB Infinity Cache (MALL) cannot stay cached between
-// the kernels that write and read them; the streaming kernels read those with
-// nontemporal loads (measured: quantize_rows [16384, 17408] 155 -> 138 us, silu_mul
-// [16384, 2 x 17408] 285 -> 261 us; at [4096, 5120], where the input fits, nontemporal
-// loads were 6% slower).
-constexpr int64_t kMallBytes = int64_t(256) << 20;
+// Cache policy of the streaming kernels (quantizers, SwiGLU, unpacking), whose output is the
+// next kernel's operand: outputs are stored through the caches unless they outgrow MI355X's
+// 256 MB Infinity Cache (MALL), and inputs past the eight 4 MB L2s, which the kernel reads
+// once, are loaded nontemporally, so that they do not push the outputs out. Measured on MI355X
+// as producer + consumer in a stream, against nontemporal stores, identical outputs:
+//   quantize_rows + fused_channel_mm: [128, 4096], N = 4096 11.9 -> 10.9 us; [64, 8704], N =
+//     5120 19.1 -> 16.8; [1536, 5120], N = 5120 56.4 -> 47.5; [2048, 17408], N = 5120 176 -> 165
+//     ([1024, 17408] -> 107.6, with nontemporal loads 107.0; [1300, 17408] 133.2 and 126.8;
+//     [16384, 5120] 374.9 and 367.9; [4096, 8704] 163.6 and 166.0);
+//   quantize_grouped4096 + grouped_summed_mm, M = 2048, N = 4096, 4 groups: 157 -> 137;
+//   silu_mul_quantize + channel_mm: [700, 2 x 17408], N = 5120 93.4 -> 83.3, with plain loads
+//     90.8; [16384, 2 x 17408], whose codes outgrow the MALL, 1335 -> 1313 with nontemporal
+//     loads and stores (1318 with cached stores).
+// The producer alone takes up to a fifth longer with cached stores (quantize_rows [2048,
+// 17408] 20 -> 23 us): they are written back when it ends.
+constexpr int64_t kL2Bytes = int64_t(32) << 20, kMallBytes = int64_t(256) << 20;
+enum StreamPolicy { kCached, kNtLoads, kNtLoadsAndStores };
+inline StreamPolicy stream_policy(int64_t in_bytes, int64_t out_bytes) {
+  if (out_bytes > kMallBytes) return kNtLoadsAndStores;
+  return in_bytes > kL2Bytes ? kNtLoads : kCached;
+}
+
+// Store by that policy.
+template <StreamPolicy kPolicy, class T>
+__device__ __forceinline__ void stream_store(T v, T* p) {
+  if constexpr (kPolicy == kNtLoadsAndStores)
+    __builtin_nontemporal_store(v, p);
+  else
+    *p = v;
+}
 
 // One 16-byte load, nontemporal when kNt.
 template <bool kNt>

@@ -11,10 +11,11 @@
 // divides only near half-integers (codes8 in ci8_device.h), with the same codes.
 //
 // Layout: one, two or four waves own a row (four past 1024 values, so a lane holds
-// at most a few 16-byte packs; eight when a few rows of 2,561..4,096 values leave most
-// CUs idle) and keep it in registers between the max reduction and the
+// at most a few 16-byte packs; eight when few and wide rows leave CUs or loads idle) and keep
+// it in registers between the max reduction and the
 // store, so HBM sees a single read of x and a single write of the codes, with 16-byte
-// loads and 8-byte stores (nontemporal outside 256..1,024 rows) fully coalesced across the wave.
+// loads and 8-byte stores (cache policy: stream_policy, ci8_device.h) fully coalesced across
+// the wave.
 #include "ci8_device.h"
 #include "launch.h"
 
@@ -33,7 +34,7 @@ __device__ __forceinline__ float wave_max(float v) {
 // kWaves waves cooperate on one row when kWaves > 1 (very wide rows).
 // Grouped: output row o reads input row (o % m) * groups + o / m ([m,g,k] -> [g,m,k]).
 // Workgroups hold four waves (1, 2 or 4 rows), or kWaves waves and one row for kWaves > 4.
-template <int kPacks, int kWaves, bool kGrouped, int kPolicy>
+template <int kPacks, int kWaves, bool kGrouped, StreamPolicy kPolicy>
 __global__ void __launch_bounds__(kWaves > 4 ? 64 * kWaves : 256) quantize_rows_vec_kernel(
     const uint16_t* __restrict__ x, int8_t* __restrict__ codes, float* __restrict__ scales,
     int rows, int k, int m, int groups) {
@@ -53,7 +54,7 @@ __global__ void __launch_bounds__(kWaves > 4 ? 64 * kWaves : 256) quantize_rows_
   for (int i = 0; i < kPacks; ++i) {
     const int col = ((i * kWaves + part) * kWave + lane) * 8;
     packed[i] = u32x4{0, 0, 0, 0};
-    if (active && col < k) packed[i] = load16<(kPolicy == 2)>(src + col);
+    if (active && col < k) packed[i] = load16<(kPolicy != kCached)>(src + col);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const uint32_t word = packed[i][j];
@@ -79,13 +80,8 @@ __global__ void __launch_bounds__(kWaves > 4 ? 64 * kWaves : 256) quantize_rows_
 #pragma unroll
   for (int i = 0; i < kPacks; ++i) {
     const int col = ((i * kWaves + part) * kWave + lane) * 8;
-    if (col < k) {
-      const u32x2 code = codes8(packed[i], scale, inv);
-      if constexpr (kPolicy >= 1)
-        __builtin_nontemporal_store(code, reinterpret_cast<u32x2*>(dst + col));
-      else
-        *reinterpret_cast<u32x2*>(dst + col) = code;
-    }
+    if (col < k)
+      stream_store<kPolicy>(codes8(packed[i], scale, inv), reinterpret_cast<u32x2*>(dst + col));
   }
 }
 
@@ -116,33 +112,17 @@ hipError_t dispatch(const void* x, int8_t* codes, float* scales, int rows, int k
   const bool vec = (reinterpret_cast<uintptr_t>(x) % 16 == 0) &&
                    (reinterpret_cast<uintptr_t>(codes) % 8 == 0) && (k % 8 == 0);
   const int packs = (k + 511) / 512;  // 16-byte packs per lane with one wave per row
-  // Inputs past the MALL's size are read with nontemporal loads (kMallBytes).
-  const bool nt = int64_t(rows) * k * 2 > kMallBytes;
-  // Codes are stored nontemporally (past the caches) except for 256 to 1,024 rows. There the
-  // GEMM that reads them next runs faster when they stay cached (measured on MI355X, graph
-  // replays of quantize_rows + fused_channel_mm, identical outputs). At M = 1024, N = 5120
-  // and K = 5120 / 8704 / 17408 the pair took 52.8 / 75.6 / 136.0 us against 59.0 / 86.3 /
-  // 153.9 us, and M = 256, N = 5120, K = 17408 took 66.7 against 70.0 us. The quantizer alone
-  // is faster with nontemporal stores ([1024, 17408]: 11.3 against 13.7 us). At 4,096 rows
-  // ([4096, 5120], N = 5120) the pair gained only 1.4 us against a 0.6 us slower quantizer,
-  // so larger inputs keep them, and so do fewer rows, whose GEMM is latency-bound.
-  // Policy (a template argument, so the store loop has no branch): 0 plain loads and
-  // stores, 1 nontemporal stores, 2 nontemporal loads and stores.
-  const int policy = nt ? 2 : (rows >= 256 && rows <= 1024 ? 0 : 1);
+  const StreamPolicy policy = stream_policy(int64_t(rows) * k * 2, int64_t(rows) * k);
 #define CI8_QW(W, P)                                                                       \
   if (packs <= (W) * (P)) {                                                                \
     constexpr int kPerBlock = (W) > 4 ? 1 : 4 / (W);                                       \
     constexpr int kThreads = (W) > 4 ? 64 * (W) : 256;                                     \
-    const int blocks = (rows + kPerBlock - 1) / kPerBlock;                                 \
-    if (policy == 2)                                                                       \
-      quantize_rows_vec_kernel<P, W, kGrouped, 2><<<blocks, kThreads, 0, stream>>>(         \
-          src, codes, scales, rows, k, m, groups);                                         \
-    else if (policy == 1)                                                                  \
-      quantize_rows_vec_kernel<P, W, kGrouped, 1><<<blocks, kThreads, 0, stream>>>(         \
-          src, codes, scales, rows, k, m, groups);                                         \
-    else                                                                                   \
-      quantize_rows_vec_kernel<P, W, kGrouped, 0><<<blocks, kThreads, 0, stream>>>(         \
-          src, codes, scales, rows, k, m, groups);                                         \
+    const auto kernel =                                                                    \
+        policy == kCached    ? quantize_rows_vec_kernel<P, W, kGrouped, kCached>           \
+        : policy == kNtLoads ? quantize_rows_vec_kernel<P, W, kGrouped, kNtLoads>          \
+                             : quantize_rows_vec_kernel<P, W, kGrouped, kNtLoadsAndStores>; \
+    kernel<<<(rows + kPerBlock - 1) / kPerBlock, kThreads, 0, stream>>>(                   \
+        src, codes, scales, rows, k, m, groups);                                           \
     return hipGetLastError();                                                              \
   }
   // Waves per row: four once a row has four packs, so each lane holds at most a few
@@ -150,15 +130,19 @@ hipError_t dispatch(const void* x, int8_t* codes, float* scales, int rows, int k
   // row): [128, 4096] 3.04 / 4.05 / 7.33, [16, 5120] 3.76 / 5.20 / 8.12, [256, 5120]
   // 3.37 / 4.31 / 7.11, [4096, 5120] 13.87 / 14.42 / 15.84: more waves keep more loads
   // in flight and let a row's stores start sooner.
-  // When the rows do not fill the chip (configs[0]'s 128 rows on 256 CUs) the op is one
+  // When the rows do not fill the chip (128 rows on 256 CUs) the op is one
   // memory latency long, and eight waves of one pack per lane shorten it a little
-  // (measured on MI355X in configs[0]'s quantize + fused_channel_mm step, 128 x 4096,
+  // (measured on MI355X in a quantize + fused_channel_mm step, 128 x 4096,
   // against four waves of two packs, same box and process: 11.80-11.86 against
   // 12.04-12.18 us on one box, 12.27-12.48 against 12.41-12.57 us on another; identical
   // codes).
-  const bool few_rows = rows <= 256;
-  if (vec && few_rows && packs > 4 && packs <= 8) {
-    CI8_QW(8, 1)
+  // Eight waves also pay for wider rows, up to 256 of them past 4,096 values and up to 1,024
+  // past 8,192 (with the GEMM that follows, four / eight waves: [16, 17408], N = 5120 24.4 /
+  // 23.7 us; [64, 8704] 17.0 / 16.8; [256, 17408] 53.2 / 52.3; [600, 17408] 89.6 / 88.3;
+  // [1024, 8704] 56.1 / 55.0; [1300, 17408] 130.7 / 133.2).
+  const bool eight = packs > 4 && rows <= (packs > 16 ? 1024 : 256);
+  if (vec && eight) {
+    CI8_QW(8, 1) CI8_QW(8, 2) CI8_QW(8, 3) CI8_QW(8, 5)
   }
   if (vec) {
     CI8_QW(1, 1) CI8_QW(2, 1) CI8_QW(4, 1) CI8_QW(4, 2) CI8_QW(4, 3) CI8_QW(4, 4)

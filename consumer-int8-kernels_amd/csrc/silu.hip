@@ -19,6 +19,8 @@
 // take an IEEE division instead, and e^-g overflows to +inf for g <= -89, giving
 // silu = -0 as in FP32 arithmetic. The quantizer's codes are bit-exact with
 // quantize_rows applied to the activations this file produces.
+#include <type_traits>
+
 #include "ci8_device.h"
 #include "launch.h"
 
@@ -102,7 +104,7 @@ __device__ __forceinline__ u32x4 swiglu8(const u32x4& gate, const u32x4& up) {
 // One row per workgroup of kWaves waves; each lane keeps kPacks packs of 8 activations
 // in registers between the row maximum and the codes. Requires k % 8 == 0,
 // k <= kPacks * kWaves * 512, x 16-byte and codes 8-byte aligned.
-template <int kPacks, int kWaves>
+template <int kPacks, int kWaves, StreamPolicy kPolicy>
 __global__ void __launch_bounds__(64 * kWaves) silu_mul_quantize_kernel(
     const uint16_t* __restrict__ x, int8_t* __restrict__ codes, float* __restrict__ scales,
     int k) {
@@ -120,8 +122,8 @@ __global__ void __launch_bounds__(64 * kWaves) silu_mul_quantize_kernel(
     const int col = ((i * kWaves + wave) * kWave + lane) * 8;
     act[i] = u32x4{0, 0, 0, 0};
     if (col < k)
-      act[i] = swiglu8(*reinterpret_cast<const u32x4*>(gate + col),
-                       *reinterpret_cast<const u32x4*>(up + col));
+      act[i] = swiglu8(load16<(kPolicy != kCached)>(gate + col),
+                       load16<(kPolicy != kCached)>(up + col));
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       amax = fmaxf(amax, fmaxf(fabsf(bf16_lo(act[i][j])), fabsf(bf16_hi(act[i][j]))));
@@ -140,21 +142,22 @@ __global__ void __launch_bounds__(64 * kWaves) silu_mul_quantize_kernel(
   for (int i = 0; i < kPacks; ++i) {
     const int col = ((i * kWaves + wave) * kWave + lane) * 8;
     if (col < k)
-      __builtin_nontemporal_store(codes8(act[i], scale, inv), reinterpret_cast<u32x2*>(dst + col));
+      stream_store<kPolicy>(codes8(act[i], scale, inv), reinterpret_cast<u32x2*>(dst + col));
   }
 }
 
 // Elementwise SwiGLU, eight outputs per lane; blockIdx.y is the row. Requires
 // k % 8 == 0 and 16-byte aligned x and out.
-template <bool kNt>
+template <StreamPolicy kPolicy>
 __global__ void __launch_bounds__(256) silu_mul_kernel(const uint16_t* __restrict__ x,
                                                        uint16_t* __restrict__ out, int k) {
   const int col = (blockIdx.x * 256 + threadIdx.x) * 8;
   if (col >= k) return;
   const int64_t row = blockIdx.y;
   const uint16_t* gate = x + row * 2 * k + col;
+  constexpr bool kNt = kPolicy != kCached;
   const u32x4 v = swiglu8(load16<kNt>(gate), load16<kNt>(gate + k));
-  __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(out + row * k + col));
+  stream_store<kPolicy>(v, reinterpret_cast<u32x4*>(out + row * k + col));
 }
 
 // Scalar fallback for rows not 16-byte aligned (silu_mul accepts any BF16 tensor).
@@ -176,12 +179,21 @@ hipError_t launch_silu_mul_quantize(const void* x, int8_t* codes, float* scales,
                                     hipStream_t stream) {
   if (m == 0) return hipSuccess;
   const auto* src = static_cast<const uint16_t*>(x);
-  // k = 8704 is 17 wave-wide packs of 512 values: 4 waves x 5 packs; k = 17408 is 34:
-  // 8 waves x 5 packs (launch-shape sweep at M = 16384).
-  if (k <= 4 * 5 * 512)
-    silu_mul_quantize_kernel<5, 4><<<m, 256, 0, stream>>>(src, codes, scales, k);
+  // k = 8704 is 17 wave-wide packs of 512 values, k = 17408 is 34: eight waves of three or
+  // five ([16, 2 x 8704] 5.1 us with four waves of five packs, 4.2 with eight of three; [256, 2
+  // x 8704] 5.6 and 5.0; [4096, 2 x 8704] level).
+  const StreamPolicy policy = stream_policy(int64_t(m) * k * 4, int64_t(m) * k);
+  auto launch = [&](auto packs) {
+    constexpr int P = decltype(packs)::value;
+    const auto kernel = policy == kCached    ? silu_mul_quantize_kernel<P, 8, kCached>
+                        : policy == kNtLoads ? silu_mul_quantize_kernel<P, 8, kNtLoads>
+                                             : silu_mul_quantize_kernel<P, 8, kNtLoadsAndStores>;
+    kernel<<<m, 512, 0, stream>>>(src, codes, scales, k);
+  };
+  if (k <= 8 * 3 * 512)
+    launch(std::integral_constant<int, 3>{});
   else
-    silu_mul_quantize_kernel<5, 8><<<m, 512, 0, stream>>>(src, codes, scales, k);
+    launch(std::integral_constant<int, 5>{});
   return hipGetLastError();
 }
 
@@ -193,12 +205,12 @@ hipError_t launch_silu_mul(const void* x, void* out, int m, int k, hipStream_t s
   const bool vec = reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(out) % 16 == 0 && k % 8 == 0;
   if (vec) {
-    // Inputs past the MALL's size are read with nontemporal loads (kMallBytes).
     const dim3 grid((k / 8 + 255) / 256, m);
-    if (count * 4 > kMallBytes)
-      silu_mul_kernel<true><<<grid, 256, 0, stream>>>(src, dst, k);
-    else
-      silu_mul_kernel<false><<<grid, 256, 0, stream>>>(src, dst, k);
+    const StreamPolicy policy = stream_policy(count * 4, count * 2);
+    const auto kernel = policy == kCached    ? silu_mul_kernel<kCached>
+                        : policy == kNtLoads ? silu_mul_kernel<kNtLoads>
+                                             : silu_mul_kernel<kNtLoadsAndStores>;
+    kernel<<<grid, 256, 0, stream>>>(src, dst, k);
   } else {
     silu_mul_scalar_kernel<<<int((count + 255) / 256), 256, 0, stream>>>(src, dst, m, k);
   }
