@@ -1,6 +1,7 @@
 // Grouped W8A8 with the per-group partials scaled and summed (grouped_summed_mm) for
-// large M on gfx950: the two-waves-per-SIMD scheme of gemm_pp.hip over the groups' K
-// stages in one stream.
+// large M on gfx950 (where grouped_ring_tile, tile_plan.h, does not expect a tile of
+// grouped_ring.hip to be faster): the two-waves-per-SIMD scheme of gemm_pp.hip over the
+// groups' K stages in one stream.
 //
 //   out[m, n] = bf16_rn( t_0 + t_1 + ... + t_{G-1} ),  FP32 additions left to right,
 //   t_g = fl( fl( float_rn(acc_g[m, n]) * sa[g, m] ) * float(sw[n]) ),

@@ -3,7 +3,8 @@
 //   out[m, n] = bf16_rn( fl( fl( float_rn(acc[m, n]) * sa[m] ) * float(sw[n]) ) )
 //   acc[m, n] = sum_k a[m, k] * w[n, k]            (exact INT32)
 //
-// for M up to a few hundred rows (csrc/fused_mm.cu:89-91 shrinks its M tile for the
+// for M up to 256 rows where gemm_choice (tile_plan.h) does not expect a tile of the ring
+// kernel (gemm_ring.hip) to be faster (csrc/fused_mm.cu:89-91 shrinks its M tile for the
 // same reason). There the GEMM is bound by moving operands, not by the MFMAs: at
 // M = 128, K = N = 4096 the 16.8 MB of weights stream from HBM once, and every
 // workgroup also reads the activation rows of its tile from L2. The large-tile kernels
