@@ -20,9 +20,9 @@ struct PPConfigT {
   static constexpr int BM = 256, BN = kBN, BK = 128;
   static constexpr int kWaves = 8, kThreads = 512;
   static constexpr int WM = 4;                        // waves along m (per group)
-  static constexpr int WN = BN / 2;                   // columns per group (112 or 80)
+  static constexpr int WN = BN / 2;                   // columns per group (112, 96, 80 or 64)
   static constexpr int TM = BM / WM / 16;             // 4 m blocks per wave
-  static constexpr int TN = WN / 16;                  // 7 (or 5) n blocks per wave
+  static constexpr int TN = WN / 16;                  // 7, 6, 5 or 4 n blocks per wave
   static constexpr int kABlocks = BM * BK / 1024;     // 32 copies of A per stage
   static constexpr int kWBlocks = BN * BK / 1024;     // 28 (or 20) copies of W per stage
   static constexpr int kCopies = kABlocks / WM;       // per A wave per stage (8)

@@ -17,8 +17,8 @@
 // weight copies): N = 5120, K = 17408: M = 1 18.9 (23.1), 5 19.6 (29.9), 16 24.4 (30.9); N =
 // 9121, K = 13168: M = 1 26.7 (32.0), 8 30.3 (43.5); N = 2560, K = 10240: M = 8 8.5 (17.0); N =
 // K = 4096: M = 5 6.2 (7.5), 16 6.6 (8.3). More slots per wave (up to 8) ran 0-5% slower
-// (fewer workgroups fit a CU), nontemporal weight copies 3-10% slower except past one round
-// of tiles. A barrier-synchronized ring with 16-row tiles (gguf_ring.hip's kernel with
+// (fewer workgroups fit a CU), nontemporal weight copies 3-10% slower up to 89 MB
+// of weights and 5-12% faster past that (gemv_stream_nontemporal, tile_plan.h). A barrier-synchronized ring with 16-row tiles (gguf_ring.hip's kernel with
 // channel scales) was slower nearly everywhere (N = 5120, K = 17408: 22.4), since its stages of
 // a few KiB cost 0.2 us each.
 #include "ci8_device.h"
@@ -29,10 +29,12 @@ namespace {
 
 constexpr int kLdsLimit = 160 * 1024;
 
-// WC: copies of W per stage (8 channels each); XC: copies of x (4 rows each: 1, 2 or 4).
-template <int WC_, int XC_>
+// WC: copies of W per stage (8 channels each); XC: copies of x (4 rows each: 1, 2 or 4); kNt:
+// W is copied nontemporally.
+template <int WC_, int XC_, bool kNt_>
 struct StreamConfig {
   static constexpr int WC = WC_, XC = XC_;
+  static constexpr int kWPolicy = kNt_ ? kBufferLoadNontemporal : 0;
   static constexpr int BN = 8 * WC, kRows = 4 * XC;
   static constexpr int TN = (WC + 1) / 2;       // 16-channel MFMA blocks (the last may be half)
   static constexpr int BK = 128;                // K values per stage
@@ -47,6 +49,12 @@ struct StreamConfig {
   static_assert(kSlots >= 3 && kWaves * TN * 1024 <= kLdsBytes, "LDS");
   static_assert((kSlots - 1) * kCopies < 64, "vmcnt");
 };
+
+template <int kPolicy>
+__device__ __forceinline__ void copy_w(__amdgpu_buffer_rsrc_t rsrc, lds_void* to, uint32_t offset,
+                                       int k0) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, to, 16, offset, k0, 0, kPolicy);
+}
 
 // Waits until at most `after` stages (kAfter at most) of kCopies copies are in flight.
 template <int kCopies, int kAfter>
@@ -116,9 +124,8 @@ __global__ void __launch_bounds__(C::kThreads) channel_gemv_stream_kernel(
     for (int q = 0; q < C::WC; ++q) {
       uint32_t off = w_off[q];
       if (!whole && k0 + w_chunk * 16 >= k) off = kOutOfRange;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          make_rsrc(w, uint32_t(n) * uint32_t(k)),
-          reinterpret_cast<lds_void*>(slot + (C::XC + q) * 1024), 16, off, k0, 0, 0);
+      copy_w<C::kWPolicy>(make_rsrc(w, uint32_t(n) * uint32_t(k)),
+                          reinterpret_cast<lds_void*>(slot + (C::XC + q) * 1024), off, k0);
     }
   };
 
@@ -218,16 +225,16 @@ hipError_t run_stream(const void* x, const int8_t* w, const void* scale, void* o
 }
 
 // The kernel of 8 WC channels per tile, or of more.
-template <int WC = 1>
+template <bool kNt, int WC = 1>
 hipError_t run_stream_width(int wc, const void* x, const int8_t* w, const void* scale, void* out,
                             int m, int n, int k, hipStream_t stream) {
   if constexpr (WC > kStreamMaxCopies) {
     return hipErrorInvalidValue;
   } else {
-    if (wc != WC) return run_stream_width<WC + 1>(wc, x, w, scale, out, m, n, k, stream);
-    if (m <= 4) return run_stream<StreamConfig<WC, 1>>(x, w, scale, out, m, n, k, stream);
-    if (m <= 8) return run_stream<StreamConfig<WC, 2>>(x, w, scale, out, m, n, k, stream);
-    return run_stream<StreamConfig<WC, 4>>(x, w, scale, out, m, n, k, stream);
+    if (wc != WC) return run_stream_width<kNt, WC + 1>(wc, x, w, scale, out, m, n, k, stream);
+    if (m <= 4) return run_stream<StreamConfig<WC, 1, kNt>>(x, w, scale, out, m, n, k, stream);
+    if (m <= 8) return run_stream<StreamConfig<WC, 2, kNt>>(x, w, scale, out, m, n, k, stream);
+    return run_stream<StreamConfig<WC, 4, kNt>>(x, w, scale, out, m, n, k, stream);
   }
 }
 
@@ -235,7 +242,9 @@ hipError_t run_stream_width(int wc, const void* x, const int8_t* w, const void* 
 
 hipError_t launch_stream_gemv(int copies, const void* x, const int8_t* w, const void* scale,
                               void* out, int m, int n, int k, hipStream_t stream) {
-  return run_stream_width(copies, x, w, scale, out, m, n, k, stream);
+  if (gemv_stream_nontemporal(n, k))
+    return run_stream_width<true>(copies, x, w, scale, out, m, n, k, stream);
+  return run_stream_width<false>(copies, x, w, scale, out, m, n, k, stream);
 }
 
 }  // namespace ci8

@@ -353,11 +353,26 @@ inline int grouped_ring_tile(int m, int n, int k, int groups, int cus, bool pers
 //     8192 15.8-16.7 against 17.4-19.3. Beyond, the span kernel is level or faster (12000 x
 //     6000, M = 9: 15.9 against 16.3; 28672 x 8192: 48.5 against 51.0), and so are the row
 //     and quad kernels at M <= 4 (17408 x 5120, M = 2: 15.6 against 18.7).
+//   Past 96 MB of weights in whole 128-byte lines, with nontemporal copies (below): M >= 9, K
+//     >= 4096 (14336 x 8192 24.0-24.1 against 28.7-31.2; 28672 x 8192 45.1-46.2 against
+//     47.7-50.1; 28672 x 4096 26.6-27.2 against 27.9-28.7) and M >= 5, K = 4224..5120 (34816
+//     x 5120 35.1-37.7 against 37.8-40.2; 24576 x 5120 25.0-28.1 against 26.9-29.1). At M =
+//     5..8 the quad kernel is faster past K = 5120 (28672 x 8192, M = 5: 41.4 against 45.9) and
+//     the span kernel at K = 4096 (28672 x 4096: 27.1 against 27.8).
 constexpr int kStreamMaxCopies = 9;
+// Whether the stream kernel copies W nontemporally: past 96 MB, in whole lines. Plain / nt:
+// 14336 x 8192, M = 9 27.0 / 24.0, 20480 x 10240, M = 1 43.2 / 39.9; 89 MB: 17408 x 5120, M =
+// 16 19.2 / 19.7; rows that start inside a line: 9121 x 13168, M = 1 27.1 / 29.5.
+inline bool gemv_stream_nontemporal(int n, int k) {
+  return k % 128 == 0 && int64_t(n) * k > int64_t(96) << 20;
+}
 inline int gemv_stream_copies(int m, int n, int k, int cus) {
   if (cus <= 0) return 0;
   const int64_t channels = (int64_t(n) + cus - 1) / cus;
-  if (!(k > 8192 || (m >= 5 && channels <= 20) || (m >= 9 && k >= 5120 && channels <= 40)))
+  const bool large = gemv_stream_nontemporal(n, k) &&
+                     ((m >= 9 && k >= 4096) || (m >= 5 && k > 4096 && k <= 5120));
+  if (!(large || k > 8192 || (m >= 5 && channels <= 20) ||
+        (m >= 9 && k >= 5120 && channels <= 40)))
     return 0;
   const int64_t rounds = (channels + 8 * kStreamMaxCopies - 1) / (8 * kStreamMaxCopies);
   return int(((int64_t(n) + cus * rounds - 1) / (cus * rounds) + 7) / 8);

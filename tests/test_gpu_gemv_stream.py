@@ -25,6 +25,8 @@ SHAPES = [
     (3, 6, 5117, 144), (3, 16, 5120, 2064), (4, 9, 8190, 5136), (5, 12, 10001, 5120),
     (6, 1, 12003, 8208), (7, 3, 14001, 8208), (8, 4, 16001, 8208), (9, 2, 18001, 8208),
     (5, 7, 19000, 8224), (3, 4, 5120, 17408),
+    # past 96 MB: nontemporal copies
+    (7, 9, 27001, 4096), (6, 5, 24501, 4224), (5, 16, 18433, 8192), (9, 12, 34817, 3072 + 1152), (6, 1, 11801, 8576),
 ]
 
 PROGRAM = r"""
@@ -49,7 +51,8 @@ def test_choices(tmp_path):
     subprocess.run([gxx, "-std=c++17", "-O1", f"-I{PKG / 'csrc'}", str(tmp_path / "plan.cpp"), "-o",
                     str(tmp_path / "plan")], check=True)
     others = [(1, 4096, 4096, 256), (4, 17408, 5120, 256), (8, 8192, 8192, 256),
-              (16, 17408, 5120, 256), (5, 512, 512, 0)]
+              (16, 17408, 5120, 256), (5, 512, 512, 0),
+              (8, 28672, 8192, 256), (8, 28672, 4096, 256), (16, 28672, 4112, 256)]
     cases = [(m, n, k, 256) for _, m, n, k in SHAPES] + others
     lines = subprocess.run([str(tmp_path / "plan"), *(str(v) for c in cases for v in c)], check=True,
                            capture_output=True, text=True).stdout.split()
