@@ -17,10 +17,10 @@
 // weight copies): N = 5120, K = 17408: M = 1 18.9 (23.1), 5 19.6 (29.9), 16 24.4 (30.9); N =
 // 9121, K = 13168: M = 1 26.7 (32.0), 8 30.3 (43.5); N = 2560, K = 10240: M = 8 8.5 (17.0); N =
 // K = 4096: M = 5 6.2 (7.5), 16 6.6 (8.3). More slots per wave (up to 8) ran 0-5% slower
-// (fewer workgroups fit a CU), nontemporal weight copies 3-10% slower up to 89 MB
-// of weights and 5-12% faster past that (gemv_stream_nontemporal, tile_plan.h). A barrier-synchronized ring with 16-row tiles (gguf_ring.hip's kernel with
-// channel scales) was slower nearly everywhere (N = 5120, K = 17408: 22.4), since its stages of
-// a few KiB cost 0.2 us each.
+// (fewer workgroups fit a CU), nontemporal weight copies 3-10% slower up to 89 MB of weights
+// and 5-12% faster past that (gemv_stream_nontemporal, tile_plan.h). A barrier-synchronized
+// ring with 16-row tiles (gguf_ring.hip's kernel with channel scales) was slower nearly
+// everywhere (N = 5120, K = 17408: 22.4), since its stages of a few KiB cost 0.2 us each.
 #include "ci8_device.h"
 #include "launch.h"
 

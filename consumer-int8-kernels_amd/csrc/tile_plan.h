@@ -280,7 +280,9 @@ constexpr int kGgufTileCount = sizeof(kGgufTiles) / sizeof(kGgufTiles[0]);
 
 // The ring tile for gguf_q8_packed_mm, or -1 where gguf_q8.hip's kernels are expected to be
 // faster: its span kernel up to M = 16 (time in channels per CU: 0.95 us per 16 channels
-// and 1024 of K at M = 1, 1.4 at M = 16, past 3.2 us), its 256- or 128-row tiles beyond
+// and 1024 of K at M = 1, 1.4 at M = 16, past 3.2 us; past 32 channels less, so there the ring
+// has to be expected 12% below: N = 5500, K = 4096, two groups, M = 11 12.0 us against 13.4; N
+// = 2234, K = 8064, four groups 19.1 against 20.8), its 256- or 128-row tiles beyond
 // (large_rows, of which it takes the one with fewer rounds). With the measured times the
 // choice is within 1% of the best kernel in the mean.
 inline int gguf_large_rows(int m, int n, int groups, int cus) {
@@ -294,6 +296,7 @@ inline int gguf_ring_tile(int m, int n, int k, int groups, int cus) {
   if (m <= 16) {
     const double channels = double((int64_t(n) * groups + cus - 1) / cus);
     best = 3.2 + channels / 16 * k / 1024 * (0.95 + 0.027 * m);
+    if (channels > 32) best *= 0.88;
   } else {
     const int rows = gguf_large_rows(m, n, groups, cus);
     best = tiled_time(tile_count(m, n, rows, 128) * groups, cus, rows == 256 ? 8.6 : 4.4,
