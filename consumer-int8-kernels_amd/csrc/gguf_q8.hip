@@ -678,9 +678,7 @@ hipError_t launch_gguf_q8_packed_mm(const void* x, const int8_t* codes, const vo
   // The ring kernel where its tiles are expected to finish first (tile_plan.h), while x's
   // and the codes' byte ranges fit a buffer's.
   const bool buffers = (int64_t(m - 1) * xs + k) * 2 <= INT32_MAX && int64_t(n) * k <= INT32_MAX;
-  if (const int tile = buffers ? gguf_ring_tile(m, n, k, groups, cus) : -1;
-      tile >= 0 &&
-      tile_count(m, n, kGgufTiles[tile].bm, kGgufTiles[tile].bn) * groups <= INT32_MAX)
+  if (const int tile = buffers ? gguf_ring_tile(m, n, k, groups, cus) : -1; tile >= 0)
     return launch_gguf_ring(tile, x, codes, scales, out, m, n, k, groups, xs, xg, stream);
   // m <= 16: the balanced-span kernel while each wave's K range holds its x fragments
   // in registers (K <= 16 ranges x 8 blocks x 64) and x's byte range fits a buffer.

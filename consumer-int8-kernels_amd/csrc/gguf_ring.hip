@@ -63,6 +63,7 @@ template <int BM_, int BN_>
 struct GgufRingConfig {
   static constexpr int BM = BM_, BN = BN_;
   static constexpr int kWaves = 8, kThreads = 64 * kWaves;
+  static_assert(kThreads == kGgufRingThreads, "tile_plan.h");
   static constexpr int WN = BM * BN >= 64 * 64 ? 2 : 1;  // waves of one K group, along n
   static constexpr int KG = kWaves / WN;                 // K groups
   static constexpr int TM = BM / 16, TN = BN / WN / 16;

@@ -278,13 +278,20 @@ constexpr RingTile kGgufTiles[] = {
     {128, 64, 6.6, 4.76}, {128, 96, 8.1, 6.50}, {128, 128, 10.0, 7.99}};
 constexpr int kGgufTileCount = sizeof(kGgufTiles) / sizeof(kGgufTiles[0]);
 
+// The most workgroups of `threads` that one launch can hold along x: HIP counts a launch's
+// work-items in 32 bits and refuses more.
+constexpr int64_t max_blocks(int threads) { return int64_t(UINT32_MAX) / threads; }
+constexpr int kGgufRingThreads = 512;
+
 // The ring tile for gguf_q8_packed_mm, or -1 where gguf_q8.hip's kernels are expected to be
 // faster: its span kernel up to M = 16 (time in channels per CU: 0.95 us per 16 channels
 // and 1024 of K at M = 1, 1.4 at M = 16, past 3.2 us; past 32 channels less, so there the ring
 // has to be expected 12% below: N = 5500, K = 4096, two groups, M = 11 12.0 us against 13.4; N
 // = 2234, K = 8064, four groups 19.1 against 20.8), its 256- or 128-row tiles beyond
 // (large_rows, of which it takes the one with fewer rounds). With the measured times the
-// choice is within 1% of the best kernel in the mean.
+// choice is within 1% of the best kernel in the mean. A tile whose
+// workgroups a launch cannot hold (M = 2097120, N = 3, K = 2048, 512 groups: 8,388,608 of 128 x
+// 64) is left out.
 inline int gguf_large_rows(int m, int n, int groups, int cus) {
   const int64_t tiles256 = tile_count(m, n, 256, 128) * groups;
   const int64_t tiles128 = tile_count(m, n, 128, 128) * groups;
@@ -305,7 +312,9 @@ inline int gguf_ring_tile(int m, int n, int k, int groups, int cus) {
   int tile = -1;
   for (int i = 0; i < kGgufTileCount; ++i) {
     const RingTile& t = kGgufTiles[i];
-    const double time = tiled_time(tile_count(m, n, t.bm, t.bn) * groups, cus, t.fixed, t.per_k, k);
+    const int64_t tiles = tile_count(m, n, t.bm, t.bn) * groups;
+    if (tiles > max_blocks(kGgufRingThreads)) continue;
+    const double time = tiled_time(tiles, cus, t.fixed, t.per_k, k);
     if (time < best) best = time, tile = i;
   }
   return tile;

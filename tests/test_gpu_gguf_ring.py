@@ -45,24 +45,49 @@ int main(int argc, char** argv) {
 """
 
 
-def test_tile_choices(tmp_path):
+@pytest.fixture(scope="module")
+def choose(tmp_path_factory):
+    """(m, n, k, groups, cus) cases -> chosen (bm, bn), (0, 0) for none; and the tile count."""
     gxx = shutil.which("g++")
     if gxx is None:
         pytest.skip("g++ not available")
-    (tmp_path / "plan.cpp").write_text(PROGRAM)
-    subprocess.run([gxx, "-std=c++17", "-O1", f"-I{PKG / 'csrc'}", str(tmp_path / "plan.cpp"), "-o",
-                    str(tmp_path / "plan")], check=True)
+    folder = tmp_path_factory.mktemp("gguf_plan")
+    (folder / "plan.cpp").write_text(PROGRAM)
+    subprocess.run([gxx, "-std=c++17", "-O1", f"-I{PKG / 'csrc'}", str(folder / "plan.cpp"), "-o",
+                    str(folder / "plan")], check=True)
+
+    def run(cases):
+        lines = subprocess.run([str(folder / "plan"), *(str(v) for c in cases for v in c)], check=True,
+                               capture_output=True, text=True).stdout.split("\n")
+        return [tuple(map(int, line.split())) for line in lines[: len(cases)]], int(lines[len(cases)])
+
+    return run
+
+
+def test_tile_choices(choose):
     # By hand: M = 2048, N = K = 4096 runs 256 tiles of 256 x 128, one round, 66.9 us, 512
     # ring tiles of 128 x 128 two of 42.0; M = 1, N = K = 4096 16 channels a CU: 7.1 against
     # 7.5 us for 256 tiles of 16 x 16; without a CU count nothing is chosen.
     by_hand = [(2048, 4096, 4096, 1, 256), (1, 4096, 4096, 1, 256), (64, 4096, 4096, 1, 0)]
     cases = [(m, n, k, g, 256) for _, m, g, n, k, _ in SHAPES] + by_hand
-    lines = subprocess.run([str(tmp_path / "plan"), *(str(v) for c in cases for v in c)], check=True,
-                           capture_output=True, text=True).stdout.split("\n")
-    got = [tuple(map(int, line.split())) for line in lines[: len(cases)]]
+    got, count = choose(cases)
     assert got[: len(SHAPES)] == [s[0] for s in SHAPES]
     assert got[len(SHAPES):] == [(0, 0)] * len(by_hand)
-    assert len({s[0] for s in SHAPES}) == int(lines[len(cases)])
+    assert len({s[0] for s in SHAPES}) == count
+
+
+def test_launches_fit_32_bit_work_item_counts(choose):
+    """HIP refuses 2^32 work-items or more along x. A tile of which a call would need that many
+    (512 threads each; the most rows the operator takes, and hundreds of groups that share x
+    through small strides) is never chosen, the largest count that fits is."""
+    m, n = 65535 * 32, 3
+    cases = [(m, n, k, g, 256) for g in (256, 511, 512, 1000, 65535) for k in (64, 1024, 2048, 4096)]
+    got, _ = choose(cases)
+    for (*_, groups, _), (bm, bn) in zip(cases, got):
+        blocks = -(-m // bm) * -(-n // bn) * groups if bm else 0
+        assert blocks * 512 < 2**32, (groups, bm, bn)
+    assert got[cases.index((m, n, 2048, 511, 256))] != (0, 0)
+    assert got[cases.index((m, n, 2048, 512, 256))] == (0, 0)
 
 
 @pytest.mark.gpu
