@@ -283,15 +283,26 @@ constexpr int kGgufTileCount = sizeof(kGgufTiles) / sizeof(kGgufTiles[0]);
 constexpr int64_t max_blocks(int threads) { return int64_t(UINT32_MAX) / threads; }
 constexpr int kGgufRingThreads = 512;
 
+// Time (us) of the span kernel (gguf_q8.hip, M <= 16) for `channels` of all groups per CU,
+// which it pads to blocks of 16, and K, which its 16 waves' ranges pad to 2, 4, 5 or 8 blocks
+// of 64 each: fitted to 208 shapes measured on MI355X (M = 1..16, N = 1024..8192, K =
+// 1024..8192, one to four groups; rms error 6%).
+inline double gguf_span_time(int m, int64_t channels, int k) {
+  const int range = (k + 1023) / 1024;
+  const int held = range <= 2 ? 2 : range <= 4 ? 4 : range <= 5 ? 5 : (range + 7) / 8 * 8;
+  return 2.15 + k / 1024.0 * (0.49 + 0.42 * double(channels) / 16) +
+         held * (0.027 * m + 0.165 * double((channels + 15) / 16));
+}
+
 // The ring tile for gguf_q8_packed_mm, or -1 where gguf_q8.hip's kernels are expected to be
-// faster: its span kernel up to M = 16 (time in channels per CU: 0.95 us per 16 channels
-// and 1024 of K at M = 1, 1.4 at M = 16, past 3.2 us; past 32 channels less, so there the ring
-// has to be expected 12% below: N = 5500, K = 4096, two groups, M = 11 12.0 us against 13.4; N
-// = 2234, K = 8064, four groups 19.1 against 20.8), its 256- or 128-row tiles beyond
-// (large_rows, of which it takes the one with fewer rounds). With the measured times the
-// choice is within 1% of the best kernel in the mean. A tile whose
-// workgroups a launch cannot hold (M = 2097120, N = 3, K = 2048, 512 groups: 8,388,608 of 128 x
-// 64) is left out.
+// faster: its span kernel up to M = 16, its 256- or 128-row tiles beyond (large_rows, of which
+// it takes the one with fewer rounds). The ring has to be expected 7% below the span kernel,
+// about the models' errors: of those 208 shapes none then ran slower by it than by the span
+// kernel beyond the spread of the runs, and the choice was 0.6% off the best kernel in the mean
+// (N = 7022, K = 1344, M = 12: 4.8 us by the span kernel, 5.7 by the ring; N = 8038, K = 2112,
+// two groups, M = 16 9.6 and 10.4; N = K = 8192, M = 1 21.2 and 14.4); past M = 16 it is 0.3%
+// off over 392. A tile whose workgroups a launch cannot hold (M = 2097120, N = 3, K = 2048, 512
+// groups: 8,388,608 of 128 x 64) is left out.
 inline int gguf_large_rows(int m, int n, int groups, int cus) {
   const int64_t tiles256 = tile_count(m, n, 256, 128) * groups;
   const int64_t tiles128 = tile_count(m, n, 128, 128) * groups;
@@ -301,9 +312,7 @@ inline int gguf_ring_tile(int m, int n, int k, int groups, int cus) {
   if (cus <= 0) return -1;
   double best;
   if (m <= 16) {
-    const double channels = double((int64_t(n) * groups + cus - 1) / cus);
-    best = 3.2 + channels / 16 * k / 1024 * (0.95 + 0.027 * m);
-    if (channels > 32) best *= 0.88;
+    best = 0.93 * gguf_span_time(m, (int64_t(n) * groups + cus - 1) / cus, k);
   } else {
     const int rows = gguf_large_rows(m, n, groups, cus);
     best = tiled_time(tile_count(m, n, rows, 128) * groups, cus, rows == 256 ? 8.6 : 4.4,
