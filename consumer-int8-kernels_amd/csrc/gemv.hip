@@ -38,10 +38,10 @@
 // 5120): it runs the products on the 4x4x4 MFMA over blocks of 4 channels so that each
 // load instruction reads 4 channels x 256 contiguous bytes, and deals the blocks to the
 // CUs round-robin so the chip streams one contiguous window.
-// The stream kernel (gemv_stream.hip) comes before all of these where gemv_stream_copies
-// (tile_plan.h) expects it to be faster and x starts on 16 bytes: K > 8192, and m >= 5 with
-// few channels a CU. So the following see K > 8192 only for an x that starts elsewhere: at m =
-// 1 while x[0:m, :] fits in 64 KiB of LDS, a second kernel copies all of x into LDS once and
+// The stream kernel (gemv_stream.hip) comes before all of these where gemv_stream_pays
+// (tile_plan.h) expects it to be faster and x starts on 16 bytes: most of K > 8192, and m >= 5
+// with few channels a CU. K > 8192 otherwise (some shapes at m <= 3, and an x that starts
+// elsewhere): while x[0:m, :] fits in 64 KiB of LDS, a kernel copies all of x into LDS once and
 // then lets every wave stream its W through a rolling window of ten 64-byte blocks with no
 // barriers at all, which removes the per-stage lock-step of the ring. Up to 160 KiB of LDS, a
 // persistent form of it runs one workgroup per CU that copies x once and walks its channel
