@@ -1241,7 +1241,8 @@ hipError_t dispatch(const int8_t* a, const void* w, const float* sa, const void*
   const bool persistent_ok =
       !kWorkspace && n % 4 == 0 && reinterpret_cast<uintptr_t>(sw) % 8 == 0;
   if (schedule == 0) {
-    const GemmChoice best = gemm_choice(m, n, k, cus, persistent_ok);
+    const GemmChoice best = gemm_choice(m, n, k, cus, persistent_ok, kWorkspace,
+                                        reinterpret_cast<uintptr_t>(out) % 16 == 0);
     if (best.ring >= 0)
       return launch_ring_gemm(best.ring, a, w, kCode, sa, sw, out, ws, m, n, k, stream);
     if constexpr (!kWorkspace)

@@ -237,19 +237,34 @@ inline double small_time(int m, int n, int k, int cus) {
 // (the small-M kernel up to kSmallMaxM, the persistent or the one-wave-per-SIMD kernel from
 // M = 1024 on) and the persistent kernel. The persistent kernel is also taken below M =
 // 1024 where its tiles fill most of a round. persistent_ok: it can run this call.
+// workspace: the INT32 products are stored too. out16: the output starts on 16 bytes.
+//
+// The times above are of BF16 outputs whose rows start on 16 bytes. What else costs time grows
+// with the outputs (us per million of them, fitted to 1600 shapes, half with N % 8 == 4 and a
+// third with products):
+//   - the persistent kernel's narrower stores where rows do not start on 16 bytes: 1.7 (M = 1018,
+//     N = 7340, K = 1088: 26.7 us, which a 128 x 128 ring tile does in 18.9);
+//   - the products: 0.85 + 0.03 per 1024 outputs of a ring tile (a round of large tiles stores
+//     them all at its end), 1.1 for the one-wave-per-SIMD kernel, which the ring has to be
+//     expected 10% below there (M = 2870, N = 3716, K = 5088: ring 120 us, that kernel 94).
 struct GemmChoice {
   int ring;
   bool persistent;
 };
-inline GemmChoice gemm_choice(int m, int n, int k, int cus, bool persistent_ok) {
+inline GemmChoice gemm_choice(int m, int n, int k, int cus, bool persistent_ok, bool workspace,
+                              bool out16 = true) {
   GemmChoice choice{-1, false};
   if (cus <= 0) return choice;
+  const double outputs = double(m) * n / 1e6;
   double best = 0.0;
   for (int i = 0; i < kRingTileCount; ++i) {
-    const double t = ring_time(kRingTiles[i], m, n, k, cus);
+    const RingTile& tile = kRingTiles[i];
+    double t = ring_time(tile, m, n, k, cus);
+    if (workspace) t += outputs * (0.85 + 0.03 * tile.bm * tile.bn / 1024);
     if (choice.ring < 0 || t < best) best = t, choice.ring = i;
   }
-  if (m <= kSmallMaxM && small_time(m, n, k, cus) <= best) return {-1, false};
+  if (m <= kSmallMaxM && small_time(m, n, k, cus) + (workspace ? 0.85 * outputs : 0.0) <= best)
+    return {-1, false};
   if (m <= kSmallOnlyMaxM) return choice;
   if (persistent_ok) {
     // Where 224-wide persistent tiles lose to 256-wide ones on rounds, another width or the
@@ -257,14 +272,16 @@ inline GemmChoice gemm_choice(int m, int n, int k, int cus, bool persistent_ok) 
     // of 256, 2.69 of 192) 237.8 -> 216.8 us; M = 2048, N = K = 8192 (one round of 256, two of
     // 128, 2% below by the model) measured 118.8 against 124.9, M = 3072, N = 5120, K = 8192
     // (240 of 256, ring 2% below) 112.6 against 119.1.
-    const double time = persistent_time(m, n, k, cus);
+    const double time = persistent_time(m, n, k, cus) +
+                        (n % 8 == 0 && out16 ? 0.0 : 1.7 * outputs);
     const double wide = 0.95 * wide_time(m, n, kPlanWideBN, k, cus);
     if (m >= 1024 && !pp_beats_wide_tiles(m, n, cus) && wide <= time)
       return wide <= best ? GemmChoice{-1, false} : choice;
     return time <= best ? GemmChoice{-1, true} : choice;
   }
-  const int wide = wide_tiles_pay(m, n, cus) ? kPlanWideBN : kPlanBN;
-  if (m >= 1024 && wide_time(m, n, wide, k, cus) <= best) return {-1, false};
+  double wide = wide_time(m, n, wide_tiles_pay(m, n, cus) ? kPlanWideBN : kPlanBN, k, cus);
+  if (workspace) wide = 0.9 * (wide + 1.1 * outputs);
+  if (m >= 1024 && wide <= best) return {-1, false};
   return choice;
 }
 

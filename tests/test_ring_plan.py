@@ -19,8 +19,9 @@ PROGRAM = r"""
 using namespace ci8;
 int main(int argc, char** argv) {
   for (int i = 1; i + 4 < argc; i += 5) {
+    const char op = argv[i + 4][0];  // f: fused or biased, w: with INT32 products, u: neither
     const GemmChoice c = gemm_choice(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]),
-                                     atoi(argv[i + 3]), atoi(argv[i + 4]) != 0);
+                                     atoi(argv[i + 3]), op == 'f', op == 'w');
     const int width = pp_width(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]),
                                atoi(argv[i + 3])).bn;
     std::printf("%d %d %d\n", c.ring < 0 ? 0 : kRingTiles[c.ring].bm,
@@ -43,7 +44,7 @@ def choose(tmp_path_factory):
                     str(folder / "plan")], check=True)
 
     def run(cases):
-        args = [str(int(v)) for case in cases for v in case]
+        args = [str(v) for case in cases for v in case]
         lines = subprocess.run([str(folder / "plan"), *args], check=True, capture_output=True,
                                text=True).stdout.split("\n")
         return [tuple(map(int, line.split())) for line in lines[: len(cases)]], int(lines[len(cases)])
@@ -52,14 +53,15 @@ def choose(tmp_path_factory):
 
 
 def test_every_ring_tile_has_a_gpu_shape(choose):
-    got, count = choose([(m, n, k, 256, True) for _, m, n, k in SHAPES])
-    for (tile, m, n, k), choice in zip(SHAPES, got):
-        assert choice == (*tile, 0), (m, n, k)
+    for op in "fw":  # cutlass_channel_mm's products come from the same tile
+        got, count = choose([(m, n, k, 256, op) for _, m, n, k in SHAPES])
+        for (tile, m, n, k), choice in zip(SHAPES, got):
+            assert choice == (*tile, 0), (m, n, k, op)
     assert len({tile for tile, *_ in SHAPES}) == count
 
 
 def test_persistent_widths_have_gpu_shapes(choose):
-    got, _ = choose([(m, n, k, 256, True) for _, m, n, k in PP_SHAPES])
+    got, _ = choose([(m, n, k, 256, "f") for _, m, n, k in PP_SHAPES])
     assert got == [(0, 0, width) for width, *_ in PP_SHAPES]
     assert {width for width, *_ in PP_SHAPES} == {224, 192, 160, 128}
 
@@ -69,23 +71,30 @@ def test_choices_by_hand(choose):
         # M = 4096, N = 17408, K = 5120: 1,248 persistent tiles, 4 + 0.75 + 0.25 * 224 / 256
         # rounds of 52.7 us = 263 us; 22 x 109 = 2,398 tiles of 192 x 160, 9.37 + rounds of
         # 38.7 us = 363 us.
-        (4096, 17408, 5120, 256, True),
+        (4096, 17408, 5120, 256, "f"),
         # M = 128, N = K = 4096: 256 small-M tiles of 64 x 32, one round: 7.9 us; 256 ring
         # tiles of 32 x 64: 8.9 us.
-        (128, 4096, 4096, 256, True),
+        (128, 4096, 4096, 256, "f"),
         # M = 1024, N = 5120, K = 17408: 256 tiles of 128 x 160, one round, 90.8 us; 92
         # persistent tiles of 224 take 0.84 of a round of 157 us, 160 of 128 0.91 of 120 us.
-        (1024, 5120, 17408, 256, True),
+        (1024, 5120, 17408, 256, "f"),
         # M = 768, N = 17408, K = 5120: 234 persistent tiles, 0.98 of a round: 53 us; ring
         # tiles take 2 rounds or more.
-        (768, 17408, 5120, 256, True),
+        (768, 17408, 5120, 256, "f"),
         # The same with an INT32 copy, which the persistent kernel does not write.
-        (768, 17408, 5120, 256, False),
+        (768, 17408, 5120, 256, "w"),
         # No CU count: the rules without a model.
-        (768, 17408, 5120, 0, True),
+        (768, 17408, 5120, 0, "f"),
         # M = 2048, N = 5120, K = 17408: 256 tiles of 256 x 160, one round, 129 us; 184 of 224
         # 0.93 of a round of 157 us, 216 of 192 0.96 of one of 141 us.
-        (2048, 5120, 17408, 256, True),
+        (2048, 5120, 17408, 256, "f"),
+        # Rows that do not start on 16 bytes: 232 persistent tiles of 128 take 12.9 us by their
+        # rounds and 12.7 more for 7.5 million outputs, 464 ring tiles of 128 x 128 19.6
+        # (measured: 26.7 us, 18.9).
+        (1018, 7340, 1088, 256, "f"),
+        # With products, 10.7 million outputs: 192 x 128 ring tiles 64 us and 17 for them, 204
+        # tiles of 224 in one round 67.7 and 11.7, 10% off (measured: 120 us, 94).
+        (2870, 3716, 5088, 256, "w"),
     ]
     got, _ = choose(cases)
     assert got[0] == (0, 0, 224)
@@ -95,3 +104,5 @@ def test_choices_by_hand(choose):
     assert got[4][0] > 0 and got[4][2] == 0
     assert got[5] == (0, 0, 0)
     assert got[6] == (0, 0, 160)
+    assert got[7][0] > 0
+    assert got[8] == (0, 0, 0)
