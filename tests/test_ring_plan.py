@@ -95,6 +95,9 @@ def test_choices_by_hand(choose):
         # With products, 10.7 million outputs: 192 x 128 ring tiles 64 us and 17 for them, 204
         # tiles of 224 in one round 67.7 and 11.7, 10% off (measured: 120 us, 94).
         (2870, 3716, 5088, 256, "w"),
+        # Level by the times, measured 4.60 and 4.54 us by the small-M kernel, 4.86 by the ring.
+        (186, 1496, 1312, 256, "f"),
+        (127, 2068, 1408, 256, "f"),
     ]
     got, _ = choose(cases)
     assert got[0] == (0, 0, 224)
@@ -106,3 +109,4 @@ def test_choices_by_hand(choose):
     assert got[6] == (0, 0, 160)
     assert got[7][0] > 0
     assert got[8] == (0, 0, 0)
+    assert got[9] == got[10] == (0, 0, 0)
