@@ -109,7 +109,7 @@ __device__ __forceinline__ void load_tile(__amdgpu_buffer_rsrc_t rsrc, lds_void*
 // through an STAGES-deep LDS ring. Returns with every vector-memory copy landed; this
 // wave's last LDS reads have been consumed by its MFMAs, but other waves may still be
 // reading the last stage, so a caller that reuses the ring must barrier first.
-template <class C, WeightCode kCode>
+template <class C>
 __device__ __forceinline__ void gemm_kloop(i32x16 (&acc)[C::TN][C::TM], const int8_t* a,
                                            const void* w,
                                            char __attribute__((address_space(3)))* lds,
@@ -159,7 +159,6 @@ __device__ __forceinline__ void gemm_kloop(i32x16 (&acc)[C::TN][C::TM], const in
         const int row = x_row0 + i * 32 + frag_row;
         xf[i] = *reinterpret_cast<const __attribute__((address_space(3))) i32x4*>(
             xs + row * C::BK + swizzle<C>(row, chunk) * 16);
-        if constexpr (kCode == WeightCode::kBiasedU8) xf[i] ^= int32_t(0x80808080u);
       }
 #pragma unroll
       for (int j = 0; j < C::TM; ++j) {
@@ -177,11 +176,10 @@ __device__ __forceinline__ void gemm_kloop(i32x16 (&acc)[C::TN][C::TM], const in
 
 }
 
-template <class C, WeightCode kCode, bool kWorkspace>
+template <class C>
 __global__ void __launch_bounds__(C::kThreads) channel_gemm_kernel(
     const int8_t* __restrict__ a, const void* __restrict__ w, const float* __restrict__ sa,
-    const uint16_t* __restrict__ sw, uint16_t* __restrict__ out, int32_t* __restrict__ ws,
-    int m, int n, int k, bool vec_n) {
+    const uint16_t* __restrict__ sw, uint16_t* __restrict__ out, int m, int n, int k, bool vec_n) {
   extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
   auto* lds = (char __attribute__((address_space(3)))*)(lds_raw);
 
@@ -212,7 +210,7 @@ __global__ void __launch_bounds__(C::kThreads) channel_gemm_kernel(
   for (int i = 0; i < C::TN; ++i)
 #pragma unroll
     for (int j = 0; j < C::TM; ++j) acc[i][j] = i32x16{};
-  gemm_kloop<C, kCode>(acc, a, w, lds, wave, lane, wave_n, wave_m, m0, n0, m, n, k);
+  gemm_kloop<C>(acc, a, w, lds, wave, lane, wave_n, wave_m, m0, n0, m, n, k);
 
   // Per-lane fragment geometry: MFMA row/col = lane % 32, K half = lane / 32.
   const int frag_row = lane & 31;
@@ -221,7 +219,7 @@ __global__ void __launch_bounds__(C::kThreads) channel_gemm_kernel(
   const int y_row0 = wave_m * (C::BM / C::WM);
 
   // Epilogue. Lane holds D[n][m] for m = lane % 32 and n = 8*r4 + 4*(lane/32) + e.
-  // vec_n: n % 4 == 0 and sw, out (and ws) aligned for 8-byte (16-byte) accesses.
+  // vec_n: n % 4 == 0 and sw and out aligned for 8-byte accesses.
   // All scale loads precede the first store (stores share the vector-memory counter).
   float row_scale[C::TM];
 #pragma unroll
@@ -256,10 +254,6 @@ __global__ void __launch_bounds__(C::kThreads) channel_gemm_kernel(
           }
           *reinterpret_cast<u32x2*>(out + base) = u32x2{pack_bf16x2(v[0], v[1]),
                                                          pack_bf16x2(v[2], v[3])};
-          if constexpr (kWorkspace)
-            *reinterpret_cast<i32x4*>(ws + base) =
-                i32x4{acc[i][j][r4 * 4 + 0], acc[i][j][r4 * 4 + 1], acc[i][j][r4 * 4 + 2],
-                      acc[i][j][r4 * 4 + 3]};
         }
       }
     }
@@ -292,10 +286,6 @@ __global__ void __launch_bounds__(C::kThreads) channel_gemm_kernel(
           }
           *reinterpret_cast<u32x2*>(out + base) = u32x2{pack_bf16x2(v[0], v[1]),
                                                          pack_bf16x2(v[2], v[3])};
-          if constexpr (kWorkspace)
-            *reinterpret_cast<i32x4*>(ws + base) =
-                i32x4{acc[i][j][r4 * 4 + 0], acc[i][j][r4 * 4 + 1], acc[i][j][r4 * 4 + 2],
-                      acc[i][j][r4 * 4 + 3]};
         }
       }
     }
@@ -316,30 +306,26 @@ __global__ void __launch_bounds__(C::kThreads) channel_gemm_kernel(
           const int64_t base = int64_t(row) * n + col;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            if (col + e < n) {
+            if (col + e < n)
               out[base + e] =
                   uint16_t(f32_to_bf16((float(acc[i][j][r4 * 4 + e]) * row_scale[j]) * sc[e]));
-              if constexpr (kWorkspace) ws[base + e] = acc[i][j][r4 * 4 + e];
-            }
           }
         }
       }
   }
 }
 
-template <class C, WeightCode kCode, bool kWorkspace>
-hipError_t run(const int8_t* a, const void* w, const float* sa, const void* sw, void* out,
-               int32_t* ws, int m, int n, int k, hipStream_t stream) {
-  auto kernel = channel_gemm_kernel<C, kCode, kWorkspace>;
-  if (const hipError_t e = prepare_lds<channel_gemm_kernel<C, kCode, kWorkspace>>(C::kLdsBytes); e != hipSuccess)
+template <class C>
+hipError_t run(const int8_t* a, const void* w, const float* sa, const void* sw, void* out, int m,
+               int n, int k, hipStream_t stream) {
+  auto kernel = channel_gemm_kernel<C>;
+  if (const hipError_t e = prepare_lds<channel_gemm_kernel<C>>(C::kLdsBytes); e != hipSuccess)
     return e;
   const int blocks = ((n + C::BN - 1) / C::BN) * ((m + C::BM - 1) / C::BM);
   const bool vec_n = n % 4 == 0 && reinterpret_cast<uintptr_t>(sw) % 8 == 0 &&
-                     reinterpret_cast<uintptr_t>(out) % 8 == 0 &&
-                     reinterpret_cast<uintptr_t>(ws) % 16 == 0;
+                     reinterpret_cast<uintptr_t>(out) % 8 == 0;
   kernel<<<blocks, C::kThreads, C::kLdsBytes, stream>>>(
-      a, w, sa, static_cast<const uint16_t*>(sw), static_cast<uint16_t*>(out), ws, m, n, k,
-      vec_n);
+      a, w, sa, static_cast<const uint16_t*>(sw), static_cast<uint16_t*>(out), m, n, k, vec_n);
   return hipGetLastError();
 }
 
@@ -572,11 +558,10 @@ struct AReloads {
   }
 };
 
-template <class C, WeightCode kCode, bool kWorkspace, bool kExactK>
+template <class C, bool kExactK>
 __global__ void __launch_bounds__(C::kThreads, 1) channel_gemm_k128_kernel(
     const int8_t* __restrict__ a, const void* __restrict__ w, const float* __restrict__ sa,
-    const uint16_t* __restrict__ sw, uint16_t* __restrict__ out, int32_t* __restrict__ ws,
-    int m, int n, int k, bool vec_n) {
+    const uint16_t* __restrict__ sw, uint16_t* __restrict__ out, int m, int n, int k, bool vec_n) {
   extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
   auto* lds = (char __attribute__((address_space(3)))*)(lds_raw);
 
@@ -679,15 +664,8 @@ __global__ void __launch_bounds__(C::kThreads, 1) channel_gemm_k128_kernel(
   // xf[1] / yf[0..TM-kSpare-1] + ysp[*] those of odd K-steps (step B).
   constexpr int kMain = C::TM - C::kSpare;
   i32x4 xf[2][C::TN], yf[C::TM], ysp[C::kSpare];
-  auto debias = [&] __device__(int buf) __attribute__((always_inline)) {
-    if constexpr (kCode == WeightCode::kBiasedU8) {
-#pragma unroll
-      for (int i = 0; i < C::TN; ++i) xf[buf][i] ^= int32_t(0x80808080u);
-    }
-  };
   // Step A: MFMAs of an even K-step; loads the odd K-step (half 1 of `slot`).
   auto step_a = [&] __device__(int slot) __attribute__((always_inline)) {
-    debias(0);
 #pragma unroll
     for (int i = 0; i < C::TN; ++i) xf[1][i] = ld(xaddr(slot, 1, i));
 #pragma unroll
@@ -714,7 +692,6 @@ __global__ void __launch_bounds__(C::kThreads, 1) channel_gemm_k128_kernel(
   // (half 0 of `next_slot`).
   auto step_b = [&] __device__(int t, int next_slot) __attribute__((always_inline)) {
     issue(t + 2);
-    debias(1);
 #pragma unroll
     for (int i = 0; i < C::TN; ++i) xf[0][i] = ld(xaddr(next_slot, 0, i));
 #pragma unroll
@@ -763,9 +740,9 @@ __global__ void __launch_bounds__(C::kThreads, 1) channel_gemm_k128_kernel(
   waitcnt<vmcnt_imm(0)>();  // padding copies of the last two steps
 #undef CI8_DMA_RSRC
 
-  store_tile16<C::TM, C::TN, kWorkspace>(acc, m0 + wave_m * (C::BM / C::WM),
-                                        n0 + wave_n * (C::BN / C::WN), m, n, sa, sw, out, ws,
-                                        vec_n);
+  store_tile16<C::TM, C::TN, false>(acc, m0 + wave_m * (C::BM / C::WM),
+                                    n0 + wave_n * (C::BN / C::WN), m, n, sa, sw, out, nullptr,
+                                    vec_n);
 }
 
 // ---------------------------------------------------------------------------------
@@ -1195,28 +1172,27 @@ hipError_t run_wlds(const int8_t* a, const void* w, const float* sa, const void*
   return run_wlds_exact<C, kCode, kWorkspace, false>(a, w, sa, sw, out, ws, m, n, k, stream);
 }
 
-template <class C, WeightCode kCode, bool kWorkspace, bool kExactK>
+template <class C, bool kExactK>
 hipError_t run_k128_exact(const int8_t* a, const void* w, const float* sa, const void* sw,
-                          void* out, int32_t* ws, int m, int n, int k, hipStream_t stream) {
-  auto kernel = channel_gemm_k128_kernel<C, kCode, kWorkspace, kExactK>;
-  if (const hipError_t e = prepare_lds<channel_gemm_k128_kernel<C, kCode, kWorkspace, kExactK>>(C::kLdsBytes); e != hipSuccess)
+                          void* out, int m, int n, int k, hipStream_t stream) {
+  auto kernel = channel_gemm_k128_kernel<C, kExactK>;
+  if (const hipError_t e = prepare_lds<channel_gemm_k128_kernel<C, kExactK>>(C::kLdsBytes);
+      e != hipSuccess)
     return e;
   const int blocks = ((n + C::BN - 1) / C::BN) * ((m + C::BM - 1) / C::BM);
   const bool vec_n = n % 4 == 0 && reinterpret_cast<uintptr_t>(sw) % 8 == 0 &&
-                     reinterpret_cast<uintptr_t>(out) % 8 == 0 &&
-                     reinterpret_cast<uintptr_t>(ws) % 16 == 0;
+                     reinterpret_cast<uintptr_t>(out) % 8 == 0;
   kernel<<<blocks, C::kThreads, C::kLdsBytes, stream>>>(
-      a, w, sa, static_cast<const uint16_t*>(sw), static_cast<uint16_t*>(out), ws, m, n, k,
-      vec_n);
+      a, w, sa, static_cast<const uint16_t*>(sw), static_cast<uint16_t*>(out), m, n, k, vec_n);
   return hipGetLastError();
 }
 
-template <class C, WeightCode kCode, bool kWorkspace>
+template <class C>
 hipError_t run_k128(const int8_t* a, const void* w, const float* sa, const void* sw, void* out,
-                    int32_t* ws, int m, int n, int k, hipStream_t stream) {
+                    int m, int n, int k, hipStream_t stream) {
   if (k % C::BK == 0)
-    return run_k128_exact<C, kCode, kWorkspace, true>(a, w, sa, sw, out, ws, m, n, k, stream);
-  return run_k128_exact<C, kCode, kWorkspace, false>(a, w, sa, sw, out, ws, m, n, k, stream);
+    return run_k128_exact<C, true>(a, w, sa, sw, out, m, n, k, stream);
+  return run_k128_exact<C, false>(a, w, sa, sw, out, m, n, k, stream);
 }
 
 // Tile configurations. All produce identical bits; they differ only in speed.
@@ -1231,53 +1207,48 @@ using WLds256 = WLdsConfig<256, 8, false>;            // 4 waves, 64x256 per wav
 // persistent kernels.
 static_assert(WLds256::BN == kPlanWideBN && WLds224::BN == kPlanBN, "tile_plan.h widths");
 
+// Schedule 0, and every call with the INT32 copy or biased weights: gemm_choice's kernel (for an
+// MI355X's 256 CUs if the device does not tell its count).
 template <WeightCode kCode, bool kWorkspace>
 hipError_t dispatch(const int8_t* a, const void* w, const float* sa, const void* sw, void* out,
-                    int32_t* ws, int m, int n, int k, int schedule, hipStream_t stream) {
-  const int cus = device_cu_count();
-  int choice = schedule;
-  // Schedule 0 first weighs the ring kernel (gemm_ring.hip) against the others (gemm_choice,
-  // tile_plan.h); what it leaves goes by the rules below.
+                    int32_t* ws, int m, int n, int k, hipStream_t stream) {
+  const int found = device_cu_count(), cus = found > 0 ? found : 256;
+  // The persistent kernel writes no INT32 copy and reads the channel scales 8 bytes at a time.
   const bool persistent_ok =
       !kWorkspace && n % 4 == 0 && reinterpret_cast<uintptr_t>(sw) % 8 == 0;
-  if (schedule == 0) {
-    const GemmChoice best = gemm_choice(m, n, k, cus, persistent_ok, kWorkspace,
-                                        reinterpret_cast<uintptr_t>(out) % 16 == 0);
-    if (best.ring >= 0)
+  const GemmChoice best = gemm_choice(m, n, k, cus, persistent_ok, kWorkspace,
+                                      reinterpret_cast<uintptr_t>(out) % 16 == 0);
+  switch (best.kernel) {
+    case GemmKernel::kSmall:
+      return launch_small_m_gemm(a, w, kCode, sa, sw, out, ws, m, n, k, cus, stream);
+    case GemmKernel::kRing:
       return launch_ring_gemm(best.ring, a, w, kCode, sa, sw, out, ws, m, n, k, stream);
-    if constexpr (!kWorkspace)
-      if (best.persistent) return launch_pp_gemm(a, w, kCode, sa, sw, out, m, n, k, stream);
-  }
-  // Schedule 0 up to M = kSmallMaxM (tile_plan.h): the small-M kernel (gemm_small.hip), or
-  // above kSmallOnlyMaxM 128 x 128 or 256 x 224 tiles where they finish sooner.
-  if (schedule == 0 && m <= kSmallMaxM) {
-    choice = mid_m_schedule(m, n, cus);
-    if (choice == 0)
-      return launch_small_m_gemm(a, w, kCode, sa, sw, out, ws, m, n, k, cus > 0 ? cus : 256,
-                                 stream);
-  }
-  if (choice == 0)
-    choice = m < 1024 || medium_tiles_pay(m, n, cus) ? 1 : (wide_tiles_pay(m, n, cus) ? 3 : 4);
-  // Without the INT32 copy, M >= 1024: the persistent two-waves-per-SIMD kernel
-  // (gemm_pp.hip) for either weight code (its epilogue reads the channel scales 8 bytes at a
-  // time) in place of the 224-wide one: per MFMA it is about 1.2x as fast.
-  if constexpr (!kWorkspace) {
-    if (schedule == 0 && m >= 1024 && choice == 4 && persistent_ok)
+    case GemmKernel::kPersistent:
       return launch_pp_gemm(a, w, kCode, sa, sw, out, m, n, k, stream);
-  }
-  switch (choice) {
-    case 5:
-      return run<Small, kCode, kWorkspace>(a, w, sa, sw, out, ws, m, n, k, stream);
-    case 1:
-      return run<Medium, kCode, kWorkspace>(a, w, sa, sw, out, ws, m, n, k, stream);
-    case 2:
-      return run<Large, kCode, kWorkspace>(a, w, sa, sw, out, ws, m, n, k, stream);
-    case 3:
+    case GemmKernel::kWide256:
       return run_wlds<WLds256, kCode, kWorkspace>(a, w, sa, sw, out, ws, m, n, k, stream);
     default:
       return run_wlds<WLds224, kCode, kWorkspace>(a, w, sa, sw, out, ws, m, n, k, stream);
-    case 6:
-      return run_k128<Pipe224, kCode, kWorkspace>(a, w, sa, sw, out, ws, m, n, k, stream);
+  }
+}
+
+// The kernels that fused_channel_mm's schedules 1 to 6 name.
+hipError_t dispatch_schedule(const int8_t* a, const void* w, const float* sa, const void* sw,
+                             void* out, int m, int n, int k, int schedule, hipStream_t stream) {
+  constexpr auto kS = WeightCode::kSigned;
+  switch (schedule) {
+    case 1:
+      return run<Medium>(a, w, sa, sw, out, m, n, k, stream);
+    case 2:
+      return run<Large>(a, w, sa, sw, out, m, n, k, stream);
+    case 3:
+      return run_wlds<WLds256, kS, false>(a, w, sa, sw, out, nullptr, m, n, k, stream);
+    case 4:
+      return run_wlds<WLds224, kS, false>(a, w, sa, sw, out, nullptr, m, n, k, stream);
+    case 5:
+      return run<Small>(a, w, sa, sw, out, m, n, k, stream);
+    default:
+      return run_k128<Pipe224>(a, w, sa, sw, out, m, n, k, stream);
   }
 }
 
@@ -1348,7 +1319,7 @@ __global__ void __launch_bounds__(C::kThreads) grouped_summed_kernel(
     for (int i = 0; i < C::TN; ++i)
 #pragma unroll
       for (int j = 0; j < C::TM; ++j) acc[i][j] = i32x16{};
-    gemm_kloop<C, WeightCode::kSigned>(acc, a + int64_t(g) * m * k, w + int64_t(g) * n * k,
+    gemm_kloop<C>(acc, a + int64_t(g) * m * k, w + int64_t(g) * n * k,
                                        lds, wave, lane, wave_n, wave_m, m0, n0, m, n, k);
     // Every wave is past its LDS reads before the next group's copies refill the ring.
     __builtin_amdgcn_s_waitcnt(lgkmcnt0_imm());
@@ -1429,13 +1400,12 @@ hipError_t launch_channel_gemm(const int8_t* a, const void* w, WeightCode code,
                                int32_t* workspace, int m, int n, int k, int schedule,
                                hipStream_t stream) {
   if (code == WeightCode::kBiasedU8)
-    return dispatch<WeightCode::kBiasedU8, false>(a, w, sa, sw, out, nullptr, m, n, k, 0,
-                                                  stream);
+    return dispatch<WeightCode::kBiasedU8, false>(a, w, sa, sw, out, nullptr, m, n, k, stream);
   if (workspace)
-    return dispatch<WeightCode::kSigned, true>(a, w, sa, sw, out, workspace, m, n, k, 0,
-                                               stream);
-  return dispatch<WeightCode::kSigned, false>(a, w, sa, sw, out, nullptr, m, n, k, schedule,
-                                              stream);
+    return dispatch<WeightCode::kSigned, true>(a, w, sa, sw, out, workspace, m, n, k, stream);
+  if (schedule != 0)
+    return dispatch_schedule(a, w, sa, sw, out, m, n, k, schedule, stream);
+  return dispatch<WeightCode::kSigned, false>(a, w, sa, sw, out, nullptr, m, n, k, stream);
 }
 
 hipError_t launch_grouped_summed_gemm(const int8_t* a, const int8_t* w, const float* sa,

@@ -103,56 +103,9 @@ inline SmallShape small_best_shape(int m, int n, int cus) {
   return best;
 }
 
-// Largest M the small-M kernel takes under schedule 0, and the M above which it competes
-// with the 128 x 128 and 256 x 224 kernels (mid_m_schedule).
+// Largest M the small-M kernel takes under schedule 0, and the M up to which only the ring
+// kernel competes with it (gemm_choice).
 constexpr int kSmallMaxM = 256, kSmallOnlyMaxM = 128;
-
-// Schedule 0 for kSmallOnlyMaxM < M <= kSmallMaxM: 0 (the small-M kernel), 1 (128 x 128
-// tiles) or 4 (256 x 224 tiles), whichever a time model of the three finishes first. The
-// model's figures are per-launch times measured on MI355X at K = 5120 (each kernel's time
-// is proportional to K, so the comparison holds at any K), conditioned graph replays,
-// identical outputs:
-//   small-M:  (its shape cost) / 13.3 us (M = 256, 64 x 32 tiles: 4 / 8 / 17 rounds took
-//             29.7 / 57.3 / 119.2 us at N = 8192 / 16384 / 34816);
-//   128x128:  35.5 us while its tiles fit one round (34.6-36.4 us from 80 to 256 tiles);
-//             past that, whole rounds plus the rest's share of a round but at least 0.37
-//             of one, as two workgroups fit a CU (M = 256: 272 / 384 / 544 tiles took
-//             48.5 / 53.2 / 86.8 us);
-//   256x224:  60 us a round (57.1-61.0 us from 23 to 156 tiles).
-// At M = 256 this takes N = 11264-24576 from 43.4-85.0 us to 34.9-53.2 us and N = 34816
-// from 119.2 to 60.3 us, and keeps the small-M kernel up to N = 8192, where it is fastest
-// (160 <= M <= 256, N from 5120 to 34816, K = 2048-17408). M <= kSmallOnlyMaxM keeps the
-// small-M kernel: its rows fill every tile of the other two, and streaming the weights
-// bounds all three alike.
-inline int mid_m_schedule(int m, int n, int cus) {
-  if (cus <= 0 || m <= kSmallOnlyMaxM || m > kSmallMaxM) return 0;
-  const double small = double(small_shape_cost(small_best_shape(m, n, cus), m, n, cus)) / 13.3;
-  const int64_t tiles128 = int64_t((m + 127) / 128) * ((n + 127) / 128);
-  double rounds128 = 1.0;
-  if (tiles128 > cus) {
-    const int64_t rest = tiles128 % cus;
-    rounds128 = double(tiles128 / cus);
-    if (rest > 0) rounds128 += rest * 100 > cus * 37 ? double(rest) / cus : 0.37;
-  }
-  const double medium = 35.5 * rounds128;
-  const int64_t tiles224 = int64_t((m + kPlanBM - 1) / kPlanBM) * ((n + kPlanBN - 1) / kPlanBN);
-  const double wide = 60.0 * double((tiles224 + cus - 1) / cus);
-  if (small <= medium && small <= wide) return 0;
-  return medium <= wide ? 1 : 4;
-}
-
-// Whether 128 x 128 tiles beat the persistent kernel at M >= 1024: when its 256 x 224 tiles
-// would keep under half the CUs busy and 128 x 128 tiles fit in one round (measured on
-// MI355X, conditioned graph replays, identical outputs: M = 1024, N = 2560 / 3072 / 2048,
-// K = 10240 / 5120 / 8192: 63.5 / 35.0 / 51.6 against 76.7 / 43.8 / 62.0 us; with more than
-// one round of 128 x 128 tiles it is not faster: M = 1024, N = 5120, K = 10240: 81.0
-// against 77.3 us, M = 2048, N = 2560: 44.4 against 44.7 us).
-inline bool medium_tiles_pay(int m, int n, int cus) {
-  if (cus <= 0 || m < 1024) return false;
-  const int64_t tiles224 = int64_t((m + kPlanBM - 1) / kPlanBM) * ((n + kPlanBN - 1) / kPlanBN);
-  const int64_t tiles128 = int64_t((m + 127) / 128) * ((n + 127) / 128);
-  return 2 * tiles224 < cus && tiles128 <= cus;
-}
 
 // Tiles of the ring kernel (gemm_ring.hip), each with the time of a round of them (one tile
 // on every CU): `fixed` + `per_k` * K / 1024 us. Fitted to 162 shapes measured on MI355X
@@ -231,12 +184,10 @@ inline double small_time(int m, int n, int k, int cus) {
   return kLaunchTime + rounds * (2.05 + 0.01146 * (s.bm + s.bn) * k / 1024);
 }
 
-// Schedule 0's first choice: the ring kernel with tile kRingTiles[ring] (ring >= 0), the
-// persistent kernel, or neither (the rules above). It goes by the times above: the ring
-// kernel is taken where its best tile is expected to beat the kernel that those rules take
-// (the small-M kernel up to kSmallMaxM, the persistent or the one-wave-per-SIMD kernel from
-// M = 1024 on) and the persistent kernel. The persistent kernel is also taken below M =
-// 1024 where its tiles fill most of a round. persistent_ok: it can run this call.
+// Schedule 0's kernel, by the times above: the ring kernel with tile kRingTiles[ring] where that
+// is expected to beat the small-M kernel (up to kSmallMaxM), the persistent kernel (persistent_ok:
+// it can run this call; above kSmallOnlyMaxM) and the one-wave-per-SIMD kernel with 256- or
+// 224-wide tiles (from M = 1024 on; 256 where the persistent kernel can run). cus > 0.
 // workspace: the INT32 products are stored too. out16: the output starts on 16 bytes.
 //
 // The times above are of BF16 outputs whose rows start on 16 bytes. What else costs time grows
@@ -247,28 +198,28 @@ inline double small_time(int m, int n, int k, int cus) {
 //   - the products: 0.85 + 0.03 per 1024 outputs of a ring tile (a round of large tiles stores
 //     them all at its end), 1.1 for the one-wave-per-SIMD kernel, which the ring has to be
 //     expected 10% below there (M = 2870, N = 3716, K = 5088: ring 120 us, that kernel 94).
+enum class GemmKernel { kSmall, kRing, kPersistent, kWide256, kWide224 };
 struct GemmChoice {
+  GemmKernel kernel;
   int ring;
-  bool persistent;
 };
 inline GemmChoice gemm_choice(int m, int n, int k, int cus, bool persistent_ok, bool workspace,
                               bool out16 = true) {
-  GemmChoice choice{-1, false};
-  if (cus <= 0) return choice;
   const double outputs = double(m) * n / 1e6;
+  GemmChoice ring{GemmKernel::kRing, 0};
   double best = 0.0;
   for (int i = 0; i < kRingTileCount; ++i) {
     const RingTile& tile = kRingTiles[i];
     double t = ring_time(tile, m, n, k, cus);
     if (workspace) t += outputs * (0.85 + 0.03 * tile.bm * tile.bn / 1024);
-    if (choice.ring < 0 || t < best) best = t, choice.ring = i;
+    if (i == 0 || t < best) best = t, ring.ring = i;
   }
   // The ring has to be expected 3% below the small-M kernel: level by the times, it was 5-7%
   // slower at the smallest calls (M = 186, N = 1496, K = 1312: 4.86 us against 4.60).
   if (m <= kSmallMaxM &&
       0.97 * (small_time(m, n, k, cus) + (workspace ? 0.85 * outputs : 0.0)) <= best)
-    return {-1, false};
-  if (m <= kSmallOnlyMaxM) return choice;
+    return {GemmKernel::kSmall, -1};
+  if (m <= kSmallOnlyMaxM) return ring;
   if (persistent_ok) {
     // Where 224-wide persistent tiles lose to 256-wide ones on rounds, another width or the
     // ring kernel has to be expected 5% below those: M = 4096, N = K = 8192 (two full rounds
@@ -279,13 +230,14 @@ inline GemmChoice gemm_choice(int m, int n, int k, int cus, bool persistent_ok, 
                         (n % 8 == 0 && out16 ? 0.0 : 1.7 * outputs);
     const double wide = 0.95 * wide_time(m, n, kPlanWideBN, k, cus);
     if (m >= 1024 && !pp_beats_wide_tiles(m, n, cus) && wide <= time)
-      return wide <= best ? GemmChoice{-1, false} : choice;
-    return time <= best ? GemmChoice{-1, true} : choice;
+      return wide <= best ? GemmChoice{GemmKernel::kWide256, -1} : ring;
+    return time <= best ? GemmChoice{GemmKernel::kPersistent, -1} : ring;
   }
-  double wide = wide_time(m, n, wide_tiles_pay(m, n, cus) ? kPlanWideBN : kPlanBN, k, cus);
+  const bool wide256 = wide_tiles_pay(m, n, cus);
+  double wide = wide_time(m, n, wide256 ? kPlanWideBN : kPlanBN, k, cus);
   if (workspace) wide = 0.9 * (wide + 1.1 * outputs);
-  if (m >= 1024 && wide <= best) return {-1, false};
-  return choice;
+  if (m < 1024 || wide > best) return ring;
+  return {wide256 ? GemmKernel::kWide256 : GemmKernel::kWide224, -1};
 }
 
 // Tiles of the GGUF ring kernel (gguf_ring.hip) with the time of a round, as kRingTiles:

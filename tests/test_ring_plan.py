@@ -20,12 +20,20 @@ using namespace ci8;
 int main(int argc, char** argv) {
   for (int i = 1; i + 4 < argc; i += 5) {
     const char op = argv[i + 4][0];  // f: fused or biased, w: with INT32 products, u: neither
-    const GemmChoice c = gemm_choice(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]),
-                                     atoi(argv[i + 3]), op == 'f', op == 'w');
-    const int width = pp_width(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]),
-                               atoi(argv[i + 3])).bn;
-    std::printf("%d %d %d\n", c.ring < 0 ? 0 : kRingTiles[c.ring].bm,
-                c.ring < 0 ? 0 : kRingTiles[c.ring].bn, c.persistent ? width : 0);
+    const int m = atoi(argv[i]), n = atoi(argv[i + 1]), k = atoi(argv[i + 2]), cus = atoi(argv[i + 3]);
+    const GemmChoice c = gemm_choice(m, n, k, cus, op == 'f', op == 'w');
+    const int width = pp_width(m, n, k, cus).bn;
+    switch (c.kernel) {
+      case GemmKernel::kSmall: std::puts("small 0 0"); break;
+      case GemmKernel::kRing:
+        std::printf("ring %d %d\n", kRingTiles[c.ring].bm, kRingTiles[c.ring].bn);
+        break;
+      case GemmKernel::kPersistent:  // width, columns of 224-wide tiles before the 160-wide ones
+        std::printf("persistent %d %d\n", width, width == kPlanBN ? pp_plan(m, n, cus).n_head : 0);
+        break;
+      case GemmKernel::kWide256: std::puts("wide 256 0"); break;
+      case GemmKernel::kWide224: std::puts("wide 224 0"); break;
+    }
   }
   std::printf("%d\n", kRingTileCount);
   return 0;
@@ -47,7 +55,8 @@ def choose(tmp_path_factory):
         args = [str(v) for case in cases for v in case]
         lines = subprocess.run([str(folder / "plan"), *args], check=True, capture_output=True,
                                text=True).stdout.split("\n")
-        return [tuple(map(int, line.split())) for line in lines[: len(cases)]], int(lines[len(cases)])
+        return [(kind, int(a), int(b)) for kind, a, b in map(str.split, lines[: len(cases)])], \
+            int(lines[len(cases)])
 
     return run
 
@@ -56,13 +65,13 @@ def test_every_ring_tile_has_a_gpu_shape(choose):
     for op in "fw":  # cutlass_channel_mm's products come from the same tile
         got, count = choose([(m, n, k, 256, op) for _, m, n, k in SHAPES])
         for (tile, m, n, k), choice in zip(SHAPES, got):
-            assert choice == (*tile, 0), (m, n, k, op)
+            assert choice == ("ring", *tile), (m, n, k, op)
     assert len({tile for tile, *_ in SHAPES}) == count
 
 
 def test_persistent_widths_have_gpu_shapes(choose):
     got, _ = choose([(m, n, k, 256, "f") for _, m, n, k in PP_SHAPES])
-    assert got == [(0, 0, width) for width, *_ in PP_SHAPES]
+    assert got == [("persistent", width, 0) for width, *_ in PP_SHAPES]
     assert {width for width, *_ in PP_SHAPES} == {224, 192, 160, 128}
 
 
@@ -83,8 +92,6 @@ def test_choices_by_hand(choose):
         (768, 17408, 5120, 256, "f"),
         # The same with an INT32 copy, which the persistent kernel does not write.
         (768, 17408, 5120, 256, "w"),
-        # No CU count: the rules without a model.
-        (768, 17408, 5120, 0, "f"),
         # M = 2048, N = 5120, K = 17408: 256 tiles of 256 x 160, one round, 129 us; 184 of 224
         # 0.93 of a round of 157 us, 216 of 192 0.96 of one of 141 us.
         (2048, 5120, 17408, 256, "f"),
@@ -100,13 +107,12 @@ def test_choices_by_hand(choose):
         (127, 2068, 1408, 256, "f"),
     ]
     got, _ = choose(cases)
-    assert got[0] == (0, 0, 224)
-    assert got[1] == (0, 0, 0)
-    assert got[2] == (128, 160, 0)
-    assert got[3] == (0, 0, 224)
-    assert got[4][0] > 0 and got[4][2] == 0
-    assert got[5] == (0, 0, 0)
-    assert got[6] == (0, 0, 160)
-    assert got[7][0] > 0
-    assert got[8] == (0, 0, 0)
-    assert got[9] == got[10] == (0, 0, 0)
+    assert got[0] == ("persistent", 224, 0)
+    assert got[1] == ("small", 0, 0)
+    assert got[2] == ("ring", 128, 160)
+    assert got[3] == ("persistent", 224, 0)
+    assert got[4][0] == "ring"
+    assert got[5] == ("persistent", 160, 0)
+    assert got[6][0] == "ring"
+    assert got[7] == ("wide", 224, 0)
+    assert got[8] == got[9] == ("small", 0, 0)
