@@ -258,12 +258,15 @@ constexpr int kGgufRingThreads = 512;
 // Time (us) of the span kernel (gguf_q8.hip, M <= 16) for `channels` of all groups per CU,
 // which it pads to blocks of 16, and K, which its 16 waves' ranges pad to 2, 4, 5 or 8 blocks
 // of 64 each: fitted to 208 shapes measured on MI355X (M = 1..16, N = 1024..8192, K =
-// 1024..8192, one to four groups; rms error 6%).
+// 1024..8192, one to four groups; rms error 6%). K past 8192 goes in chunks, about 5% more; past
+// 128 channels a CU, which the chunks' partial sums do not fit, the tile kernel takes twice as
+// long (N = 11877, K = 8704, four groups, M = 3: 136 us, the ring 80).
 inline double gguf_span_time(int m, int64_t channels, int k) {
   const int range = (k + 1023) / 1024;
   const int held = range <= 2 ? 2 : range <= 4 ? 4 : range <= 5 ? 5 : (range + 7) / 8 * 8;
-  return 2.15 + k / 1024.0 * (0.49 + 0.42 * double(channels) / 16) +
-         held * (0.027 * m + 0.165 * double((channels + 15) / 16));
+  const double time = 2.15 + k / 1024.0 * (0.49 + 0.42 * double(channels) / 16) +
+                      held * (0.027 * m + 0.165 * double((channels + 15) / 16));
+  return k <= 8192 ? time : channels <= 128 ? 1.05 * time : 2 * time;
 }
 
 // The ring tile for gguf_q8_packed_mm, or -1 where gguf_q8.hip's kernels are expected to be

@@ -74,6 +74,9 @@ def test_tile_choices(choose):
             (1, 6023, 4992, 1, 256), (16, 8038, 2112, 2, 256), (6, 8168, 2240, 1, 256)]
     by_hand = [(2048, 4096, 4096, 1, 256), (1, 4096, 4096, 1, 256), (64, 4096, 4096, 1, 0), *span]
     cases = [(m, n, k, g, 256) for _, m, g, n, k, _ in SHAPES] + by_hand
+    # K > 8192 (us, the other kernels / ring): 135.6 / 80.1, 139.3 / 68.6, 59.7 / 48.9.
+    long_k = [(3, 11877, 8704, 4, 256), (1, 8674, 9152, 4, 256), (5, 12024, 9600, 2, 256)]
+    assert choose(long_k)[0] == [(16, 32)] * 3
     got, count = choose(cases)
     assert got[: len(SHAPES)] == [s[0] for s in SHAPES]
     assert got[len(SHAPES):] == [(0, 0)] * len(by_hand)
