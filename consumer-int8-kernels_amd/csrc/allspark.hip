@@ -13,11 +13,11 @@
 // the lanes of a wave take consecutive tiles, so together they read 4 KiB of one packed
 // row), rebuilds the four output rows' 16-byte pieces with byte selects and a XOR of
 // 0x80 per byte, and stores them; consecutive lanes write consecutive 16-byte pieces of
-// each output row (stored through the caches while the layer fits the MALL, stream_policy
-// in ci8_device.h: the GEMM that follows reads it; M = 256, N = 7168, K = 5120 with quantizer
-// and GEMM 40.6 -> 36.7 us, N = 17408 80.2 -> 75.4, though the kernel alone takes 14.2 for
-// 13.6 and 38.5 for 30.9). Rows at or beyond n (the last group when n % 32 == 16) are
-// neither stored nor their bytes used. Pure data movement: HBM-bound at 2 bytes per weight.
+// each output row, by stream_policy.h: the GEMM that follows reads it (M = 256, N = 7168, K =
+// 5120 with quantizer and GEMM 40.1 us with nontemporal stores, 36.3 with plain ones, though the
+// kernel alone takes 14.2 and 14.7). Rows at or beyond n (the last group when n % 32
+// == 16) are neither stored nor their bytes used. Pure data movement: HBM-bound at 2 bytes per
+// weight.
 #include "ci8_device.h"
 #include "launch.h"
 
@@ -60,9 +60,9 @@ __global__ void __launch_bounds__(256) unpack_allspark_kernel(
   for (int q = 0; q < 4; ++q) {
     const int row = first + 8 * q;
     if (row < n)
-      stream_store<kPolicy>(
-          restore_piece(chunk[0][q], chunk[1][q], chunk[2][q], chunk[3][q]),
-          reinterpret_cast<u32x4*>(weight + int64_t(row) * k + int64_t(tile) * 16));
+      stream_store<kPolicy>(  // the layer is at most INT_MAX bytes
+          restore_piece(chunk[0][q], chunk[1][q], chunk[2][q], chunk[3][q]), weight,
+          uint32_t(n) * uint32_t(k), uint32_t(row) * uint32_t(k) + uint32_t(tile) * 16);
   }
   if (tile == 0) {
 #pragma unroll
@@ -83,14 +83,13 @@ hipError_t launch_unpack_allspark(const uint8_t* packed, const void* packed_scal
   const auto* ps = static_cast<const uint16_t*>(packed_scales);
   auto* s = static_cast<uint16_t*>(scales);
   const bool vec = reinterpret_cast<uintptr_t>(packed) % 16 == 0;
-  const bool nt = stream_policy(0, int64_t(n) * k) == kNtLoadsAndStores;
+  // Plain stores while the MALL holds the packed and the restored layer.
   auto go = [&](auto kernel) { kernel<<<grid, 256, 0, stream>>>(packed, ps, weight, s, n, k); };
-  if (vec)
-    go(nt ? unpack_allspark_kernel<true, kNtLoadsAndStores>
-          : unpack_allspark_kernel<true, kCached>);
+  if (2 * int64_t(n) * k > kMallBytes)
+    go(vec ? unpack_allspark_kernel<true, kNtLoadsAndStores>
+           : unpack_allspark_kernel<false, kNtLoadsAndStores>);
   else
-    go(nt ? unpack_allspark_kernel<false, kNtLoadsAndStores>
-          : unpack_allspark_kernel<false, kCached>);
+    go(vec ? unpack_allspark_kernel<true, kCached> : unpack_allspark_kernel<false, kCached>);
   return hipGetLastError();
 }
 

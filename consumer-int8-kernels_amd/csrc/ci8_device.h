@@ -7,6 +7,7 @@
 #include <atomic>
 
 #include "lds_budget.h"
+#include "stream_policy.h"
 
 namespace ci8 {
 
@@ -84,37 +85,6 @@ __device__ __forceinline__ u32x2 codes8(const u32x4& packed, float scale, float 
   return out;
 }
 
-// Cache policy of the streaming kernels (quantizers, SwiGLU, unpacking), whose output is the
-// next kernel's operand: outputs are stored through the caches unless they outgrow MI355X's
-// 256 MB Infinity Cache (MALL), and inputs past the eight 4 MB L2s, which the kernel reads
-// once, are loaded nontemporally, so that they do not push the outputs out. Measured on MI355X
-// as producer + consumer in a stream, against nontemporal stores, identical outputs:
-//   quantize_rows + fused_channel_mm: [128, 4096], N = 4096 11.9 -> 10.9 us; [64, 8704], N =
-//     5120 19.1 -> 16.8; [1536, 5120], N = 5120 56.4 -> 47.5; [2048, 17408], N = 5120 176 -> 165
-//     ([1024, 17408] -> 107.6, with nontemporal loads 107.0; [1300, 17408] 133.2 and 126.8;
-//     [16384, 5120] 374.9 and 367.9; [4096, 8704] 163.6 and 166.0);
-//   quantize_grouped4096 + grouped_summed_mm, M = 2048, N = 4096, 4 groups: 157 -> 137;
-//   silu_mul_quantize + channel_mm: [700, 2 x 17408], N = 5120 93.4 -> 83.3, with plain loads
-//     90.8; [16384, 2 x 17408], whose codes outgrow the MALL, 1335 -> 1313 with nontemporal
-//     loads and stores (1318 with cached stores).
-// The producer alone takes up to a fifth longer with cached stores (quantize_rows [2048,
-// 17408] 20 -> 23 us): they are written back when it ends.
-constexpr int64_t kL2Bytes = int64_t(32) << 20, kMallBytes = int64_t(256) << 20;
-enum StreamPolicy { kCached, kNtLoads, kNtLoadsAndStores };
-inline StreamPolicy stream_policy(int64_t in_bytes, int64_t out_bytes) {
-  if (out_bytes > kMallBytes) return kNtLoadsAndStores;
-  return in_bytes > kL2Bytes ? kNtLoads : kCached;
-}
-
-// Store by that policy.
-template <StreamPolicy kPolicy, class T>
-__device__ __forceinline__ void stream_store(T v, T* p) {
-  if constexpr (kPolicy == kNtLoadsAndStores)
-    __builtin_nontemporal_store(v, p);
-  else
-    *p = v;
-}
-
 // One 16-byte load, nontemporal when kNt.
 template <bool kNt>
 __device__ __forceinline__ u32x4 load16(const void* p) {
@@ -135,6 +105,29 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, ui
 }
 // An offset past every valid buffer (buffers are limited to INT_MAX bytes).
 constexpr uint32_t kOutOfRange = 0x80000000u;
+
+// Cache-policy operand of a buffer store that writes through the L2 (the sc1 bit: device
+// scope): the line is not left dirty.
+constexpr int kBufferStoreWriteThrough = 16;
+
+// Store of 8 or 16 bytes at byte offset `at` of the `bytes` bytes at `base` by the policy.
+template <StreamPolicy kPolicy, class T>
+__device__ __forceinline__ void stream_store(T v, void* base, uint32_t bytes, uint32_t at) {
+  static_assert(sizeof(T) == 8 || sizeof(T) == 16);
+  T* p = reinterpret_cast<T*>(static_cast<char*>(base) + at);
+  if constexpr (kPolicy == kCached)
+    *p = v;
+  else if constexpr (kPolicy == kNtLoadsAndStores)
+    __builtin_nontemporal_store(v, p);
+  else if constexpr (sizeof(T) == 8)
+    __builtin_amdgcn_raw_buffer_store_b64(v, make_rsrc(base, bytes), at, 0,
+                                          kBufferStoreWriteThrough);
+  else
+    __builtin_amdgcn_raw_buffer_store_b128(v, make_rsrc(base, bytes), at, 0,
+                                           kBufferStoreWriteThrough);
+}
+// Whether the policy's loads are nontemporal.
+constexpr bool nt_loads(StreamPolicy policy) { return policy >= kNtLoads; }
 
 // A kernel as a type, for launch helpers that take several kernels of one signature.
 template <auto Kernel>

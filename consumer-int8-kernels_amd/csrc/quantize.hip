@@ -14,7 +14,7 @@
 // at most a few 16-byte packs; eight when few and wide rows leave CUs or loads idle) and keep
 // it in registers between the max reduction and the
 // store, so HBM sees a single read of x and a single write of the codes, with 16-byte
-// loads and 8-byte stores (cache policy: stream_policy, ci8_device.h) fully coalesced across
+// loads and 8-byte stores (cache policy: stream_policy.h) fully coalesced across
 // the wave.
 #include "ci8_device.h"
 #include "launch.h"
@@ -54,7 +54,7 @@ __global__ void __launch_bounds__(kWaves > 4 ? 64 * kWaves : 256) quantize_rows_
   for (int i = 0; i < kPacks; ++i) {
     const int col = ((i * kWaves + part) * kWave + lane) * 8;
     packed[i] = u32x4{0, 0, 0, 0};
-    if (active && col < k) packed[i] = load16<(kPolicy != kCached)>(src + col);
+    if (active && col < k) packed[i] = load16<nt_loads(kPolicy)>(src + col);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const uint32_t word = packed[i][j];
@@ -76,12 +76,12 @@ __global__ void __launch_bounds__(kWaves > 4 ? 64 * kWaves : 256) quantize_rows_
   const float scale = fmaxf(amax / 127.f, 1e-20f);
   const float inv = 1.f / scale;
   if (part == 0 && lane == 0) scales[out_row] = scale;
-  int8_t* dst = codes + int64_t(out_row) * k;
+  // Codes are at most INT_MAX bytes.
+  const uint32_t bytes = uint32_t(rows) * uint32_t(k), at = uint32_t(out_row) * uint32_t(k);
 #pragma unroll
   for (int i = 0; i < kPacks; ++i) {
     const int col = ((i * kWaves + part) * kWave + lane) * 8;
-    if (col < k)
-      stream_store<kPolicy>(codes8(packed[i], scale, inv), reinterpret_cast<u32x2*>(dst + col));
+    if (col < k) stream_store<kPolicy>(codes8(packed[i], scale, inv), codes, bytes, at + col);
   }
 }
 
@@ -112,15 +112,15 @@ hipError_t dispatch(const void* x, int8_t* codes, float* scales, int rows, int k
   const bool vec = (reinterpret_cast<uintptr_t>(x) % 16 == 0) &&
                    (reinterpret_cast<uintptr_t>(codes) % 8 == 0) && (k % 8 == 0);
   const int packs = (k + 511) / 512;  // 16-byte packs per lane with one wave per row
-  const StreamPolicy policy = stream_policy(int64_t(rows) * k * 2, int64_t(rows) * k);
+  const StreamPolicy policy =
+      stream_policy(int64_t(rows) * k * 2, int64_t(rows) * k, kQuantizeWriteThrough);
 #define CI8_QW(W, P)                                                                       \
   if (packs <= (W) * (P)) {                                                                \
     constexpr int kPerBlock = (W) > 4 ? 1 : 4 / (W);                                       \
     constexpr int kThreads = (W) > 4 ? 64 * (W) : 256;                                     \
-    const auto kernel =                                                                    \
-        policy == kCached    ? quantize_rows_vec_kernel<P, W, kGrouped, kCached>           \
-        : policy == kNtLoads ? quantize_rows_vec_kernel<P, W, kGrouped, kNtLoads>          \
-                             : quantize_rows_vec_kernel<P, W, kGrouped, kNtLoadsAndStores>; \
+    const auto kernel = with_policy(policy, [](auto p) {                                   \
+      return quantize_rows_vec_kernel<P, W, kGrouped, decltype(p)::value>;                 \
+    });                                                                                    \
     kernel<<<(rows + kPerBlock - 1) / kPerBlock, kThreads, 0, stream>>>(                   \
         src, codes, scales, rows, k, m, groups);                                           \
     return hipGetLastError();                                                              \

@@ -122,8 +122,8 @@ __global__ void __launch_bounds__(64 * kWaves) silu_mul_quantize_kernel(
     const int col = ((i * kWaves + wave) * kWave + lane) * 8;
     act[i] = u32x4{0, 0, 0, 0};
     if (col < k)
-      act[i] = swiglu8(load16<(kPolicy != kCached)>(gate + col),
-                       load16<(kPolicy != kCached)>(up + col));
+      act[i] = swiglu8(load16<nt_loads(kPolicy)>(gate + col),
+                       load16<nt_loads(kPolicy)>(up + col));
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       amax = fmaxf(amax, fmaxf(fabsf(bf16_lo(act[i][j])), fabsf(bf16_hi(act[i][j]))));
@@ -137,12 +137,12 @@ __global__ void __launch_bounds__(64 * kWaves) silu_mul_quantize_kernel(
   const float scale = fmaxf(amax / 127.f, 1e-20f);
   const float inv = 1.f / scale;
   if (threadIdx.x == 0) scales[row] = scale;
-  int8_t* dst = codes + row * k;
+  // Codes are at most INT_MAX bytes.
+  const uint32_t bytes = gridDim.x * uint32_t(k), at = blockIdx.x * uint32_t(k);
 #pragma unroll
   for (int i = 0; i < kPacks; ++i) {
     const int col = ((i * kWaves + wave) * kWave + lane) * 8;
-    if (col < k)
-      stream_store<kPolicy>(codes8(act[i], scale, inv), reinterpret_cast<u32x2*>(dst + col));
+    if (col < k) stream_store<kPolicy>(codes8(act[i], scale, inv), codes, bytes, at + col);
   }
 }
 
@@ -155,9 +155,11 @@ __global__ void __launch_bounds__(256) silu_mul_kernel(const uint16_t* __restric
   if (col >= k) return;
   const int64_t row = blockIdx.y;
   const uint16_t* gate = x + row * 2 * k + col;
-  constexpr bool kNt = kPolicy != kCached;
+  constexpr bool kNt = nt_loads(kPolicy);
   const u32x4 v = swiglu8(load16<kNt>(gate), load16<kNt>(gate + k));
-  stream_store<kPolicy>(v, reinterpret_cast<u32x4*>(out + row * k + col));
+  // The output is at most INT_MAX bytes.
+  stream_store<kPolicy>(v, out, gridDim.y * uint32_t(k) * 2,
+                        (blockIdx.y * uint32_t(k) + uint32_t(col)) * 2);
 }
 
 // Scalar fallback for rows not 16-byte aligned (silu_mul accepts any BF16 tensor).
@@ -182,12 +184,12 @@ hipError_t launch_silu_mul_quantize(const void* x, int8_t* codes, float* scales,
   // k = 8704 is 17 wave-wide packs of 512 values, k = 17408 is 34: eight waves of three or
   // five ([16, 2 x 8704] 5.1 us with four waves of five packs, 4.2 with eight of three; [256, 2
   // x 8704] 5.6 and 5.0; [4096, 2 x 8704] level).
-  const StreamPolicy policy = stream_policy(int64_t(m) * k * 4, int64_t(m) * k);
+  const StreamPolicy policy =
+      stream_policy(int64_t(m) * k * 4, int64_t(m) * k, kQuantizeWriteThrough);
   auto launch = [&](auto packs) {
     constexpr int P = decltype(packs)::value;
-    const auto kernel = policy == kCached    ? silu_mul_quantize_kernel<P, 8, kCached>
-                        : policy == kNtLoads ? silu_mul_quantize_kernel<P, 8, kNtLoads>
-                                             : silu_mul_quantize_kernel<P, 8, kNtLoadsAndStores>;
+    const auto kernel = with_policy(
+        policy, [](auto p) { return silu_mul_quantize_kernel<P, 8, decltype(p)::value>; });
     kernel<<<m, 512, 0, stream>>>(src, codes, scales, k);
   };
   if (k <= 8 * 3 * 512)
@@ -206,10 +208,8 @@ hipError_t launch_silu_mul(const void* x, void* out, int m, int k, hipStream_t s
                    reinterpret_cast<uintptr_t>(out) % 16 == 0 && k % 8 == 0;
   if (vec) {
     const dim3 grid((k / 8 + 255) / 256, m);
-    const StreamPolicy policy = stream_policy(count * 4, count * 2);
-    const auto kernel = policy == kCached    ? silu_mul_kernel<kCached>
-                        : policy == kNtLoads ? silu_mul_kernel<kNtLoads>
-                                             : silu_mul_kernel<kNtLoadsAndStores>;
+    const auto kernel = with_policy(stream_policy(count * 4, count * 2, kSiluWriteThrough),
+                                    [](auto p) { return silu_mul_kernel<decltype(p)::value>; });
     kernel<<<grid, 256, 0, stream>>>(src, dst, k);
   } else {
     silu_mul_scalar_kernel<<<int((count + 255) / 256), 256, 0, stream>>>(src, dst, m, k);
