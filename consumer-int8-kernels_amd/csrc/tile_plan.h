@@ -339,20 +339,24 @@ inline int grouped_ring_tile(int m, int n, int k, int groups, int cus, bool pers
 
 // channel_gemv: 8-channel copies per stage of the stream kernel (gemv_stream.hip) that fill
 // the CUs in as few rounds of one tile each as its widest tile allows, or 0 where gemv.hip's
-// kernels are faster. Measured on MI355X at 2200 drawn shapes, M = 1..16 (stream against those,
+// kernels are faster. Measured on MI355X at 2563 drawn shapes, M = 1..16 (stream against those,
 // us; "lines": rows of whole 128-byte lines, K % 128 == 0, of which the stream kernel reads no
 // line twice):
-//   K > 8192, M >= 4: everywhere (5120 x 17408: 19.6-24.4 against 29.9-30.9; 2560 x 10240, M =
-//     8: 8.5 against 17.0). M <= 3: with lines (5120 x 17408, M = 1: 18.9 against 23.1), but at M
-//     <= 2 not where 16-channel workgroups, one or two a CU, fill the chip for the resident kernel
-//     (3755 x 8832, M = 1: 8.8 against 8.2; 7846 x 9984, M = 2: 16.2 against 15.2). Without lines
-//     up to 79 channels a CU (M = 2 beyond: 5% slower) and at M = 1 from 17 to 48 (9121 x 13168:
-//     26.7 against 32.0; 2128 x 14688: 10.0 against 9.6, 26801 x 9280: 55.1 against 47.2).
+//   K > 8192: M >= 3 everywhere (5120 x 17408, M = 5: 19.6 against 29.9; 2560 x 10240, M = 8: 8.5
+//     against 17.0). M <= 2: with lines (5120 x 17408, M = 1: 18.9 against 23.1), but not where the
+//     resident kernel's 16-channel workgroups, one or two a CU, fill the chip (3755 x 8832, M = 1:
+//     8.8 against 8.2; 7846 x 9984, M = 2: 16.2 against 15.2; two a CU past K = 12000 the stream
+//     again: 6352 x 17408, M = 2, with its first half 64.0 against 70.7). Without lines, M = 2 up
+//     to 79 channels a CU (beyond 4% slower) and M = 1 from 17 to 48 (9121 x 13168: 26.7 against
+//     32.0; 2128 x 14688: 10.0 against 9.6, 26801 x 9280: 55.1 against 47.2).
 //   M >= 5, up to 16 channels a CU: with lines everywhere (4096 x 4096: 6.2-6.6 against 7.5-8.3).
-//     Without, from K = 2048 on (9 of 50 shapes below ran 4-9% slower: 1684 x 1040, M = 10 3.4
-//     against 3.1), and at M <= 7 up to K = 7168 (2481 x 7824, M = 5: 8.7 against 8.2). Up to 20
-//     channels with lines (5120 x 5120: 8.2-9.4 against 8.5-10.9; without, 24 computed for 17 to
-//     20: 4839 x 1808, M = 14 5.6 against 4.9).
+//     Without, from K = 2048 on, at M <= 7 up to K = 7168 (2481 x 7824, M = 5: 8.7 against 8.2),
+//     and below where rows are whole half lines (1866 x 1984, M = 8: 3.5 against 3.7; otherwise 31
+//     of 71 shapes ran 2-8% slower: 1684 x 1040, M = 10 3.4 against 3.1).
+//   17 to 20 channels a CU (24 computed): with lines up to 19, or from K = 5120 on (5120 x 5120:
+//     8.2-9.4 against 8.5-10.9; 5036 x 3456, M = 9: 7.8 against 7.5); without, M >= 13 from 18
+//     channels and K = 5120 on (5047 x 5568, M = 14: 10.4 against 11.7; 4839 x 1808, M = 14: 5.6
+//     against 4.9).
 //   Up to 40 channels a CU, K >= 5120: M >= 9 with lines (7168 x 5120 9.8-9.9 against 9.8-11.4,
 //     8192 x 8192 15.8-16.7 against 17.4-19.3), M >= 13 without (8630 x 7056, M = 11: 15.8
 //     against 15.3). Beyond, the span kernel is level or faster (12000 x 6000, M = 9: 15.9
@@ -364,8 +368,8 @@ inline int grouped_ring_tile(int m, int n, int k, int groups, int cus, bool pers
 //     37.8-40.2; 24576 x 5120 25.0-28.1 against 26.9-29.1). At M = 5..8 the quad kernel is faster
 //     past K = 5120 (28672 x 8192, M = 5: 41.4 against 45.9) and the span kernel at K = 4096
 //     (28672 x 4096: 27.1 against 27.8).
-// Of those shapes 37 are slower than by gemv.hip's kernels by more than 2% (188 with K > 8192, M
-// >= 5 up to 20 channels, and M >= 9, K >= 5120 up to 40 channels whatever K's lines).
+// Of 363 shapes drawn from the operator's range 5 are more than 2.5% slower than by gemv.hip's
+// kernels (45 with every K > 8192, M >= 5 up to 20 channels, and M >= 9, K >= 5120 up to 40).
 constexpr int kStreamMaxCopies = 9;
 // Whether the stream kernel copies W nontemporally: past 96 MB, in whole lines. Plain / nt:
 // 14336 x 8192, M = 9 27.0 / 24.0, 20480 x 10240, M = 1 43.2 / 39.9; 89 MB: 17408 x 5120, M =
@@ -378,14 +382,15 @@ inline bool gemv_stream_pays(int m, int64_t channels, int n, int k) {
   if (gemv_stream_nontemporal(n, k) && ((m >= 9 && k >= 4096) || (m >= 5 && k > 4096 && k <= 5120)))
     return true;
   if (k > 8192) {
-    if (m >= 4) return true;
-    if (!lines) return m >= 2 ? channels < 80 : channels > 16 && channels <= 48;
-    return m == 3 || !((channels > 8 && channels <= 16) || (channels > 24 && channels <= 32));
+    if (m >= 3) return true;
+    if (!lines) return m == 2 ? channels < 80 : channels > 16 && channels <= 48;
+    return !(m == 1 && channels > 8 && channels <= 16) &&
+           !(channels > 24 && channels <= 32 && k < 12000);
   }
   if (m < 5) return false;
-  if (channels <= 16) return lines || (k >= 2048 && (m >= 8 || k < 7168));
-  if (channels <= 20 && lines) return true;
-  return channels <= 40 && k >= 5120 && m >= (lines ? 9 : 13) && (lines || channels > 20);
+  if (channels <= 16) return lines || (k >= 2048 ? m >= 8 || k < 7168 : k % 64 == 0);
+  if (lines && (channels <= 19 || (channels <= 20 && k >= 5120))) return true;
+  return channels <= 40 && k >= 5120 && (lines ? m >= 9 : m >= 13 && channels >= 18);
 }
 inline int gemv_stream_copies(int m, int n, int k, int cus) {
   if (cus <= 0) return 0;

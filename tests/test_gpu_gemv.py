@@ -62,15 +62,25 @@ def test_decode_shape_full_size(ops, m):
     check_gemv(bf16_bits(out), x_bits, w, s_bits)
 
 
-@pytest.mark.parametrize("m,n,k", [(12, 1000, 5104), (10, 4100, 5120), (14, 250, 5120),
-                                   (9, 17, 8192), (10, 16 * 256 * 3 + 16, 5120),
-                                   (7, 300, 5120), (16, 36869, 2048), (5, 2000, 4096),
-                                   (2, 16 * 256 * 9 + 5, 1024), (1, 17408, 5120)])
+# Shapes that the stream kernel (gemv_stream.hip) leaves to the kernels named; the choice is
+# checked on the CPU by tests/test_gpu_gemv_stream.py. x ranges of 2, 4, 5 and 8 blocks of 64 a
+# wave (SPAN), 4 to 8 (QUAD).
+SPAN_SHAPES = [(9, 17, 2032), (12, 1000, 2000), (16, 36869, 2048), (2, 16 * 256 * 9 + 5, 1024),
+               (9, 12001, 4080), (5, 5200, 4096), (10, 16 * 256 * 3 + 16, 5120),
+               (10, 10300, 5104), (6, 10001, 5120), (9, 12001, 6000), (9, 12001, 8176)]
+QUAD_SHAPES = [(2, 4096, 4096), (3, 1001, 4112), (4, 33000, 4096), (5, 20002, 6144),
+               (7, 9003, 6160), (8, 9001, 7168), (8, 9001, 8192), (6, 9002, 8176), (6, 517, 8176),
+               (2, 17408, 5120)]
+RESIDENT_SHAPES = [(1, 3755, 8832), (2, 7846, 9984), (1, 26801, 9280), (1, 2174, 14160)]
+
+
+@pytest.mark.parametrize("m,n,k", SPAN_SHAPES + [(1, 17408, 5120)])
 def test_balanced_spans(ops, m, n, k):
     """K <= 8192 (m >= 2) runs one workgroup per CU over equal channel spans (N = 17408:
-    68 per CU): fewer channels than CUs x 16, spans that end inside a block of 16, more
-    than 8 blocks per span (two partial-sum batches), every x-register configuration (K
-    ranges of 2, 4, 5 and 8 blocks of 64) and a K tail; m = 1 takes the row kernel."""
+    68 per CU) where neither the stream nor the quad-block kernel is faster: fewer channels
+    than CUs x 16, spans that end inside a block of 16, more than 8 blocks per span (two
+    partial-sum batches), every x-register configuration (K ranges of 2, 4, 5 and 8 blocks of
+    64) and K tails; m = 1 takes the row kernel."""
     rng = np.random.default_rng(m * 7 + n + k)
     x_bits = randn_bf16(rng, (m, k))
     w = rng.integers(-128, 128, (n, k)).astype(np.int8)
@@ -81,15 +91,14 @@ def test_balanced_spans(ops, m, n, k):
     check_gemv(bf16_bits(out), x_bits, w, s_bits)
 
 
-@pytest.mark.parametrize("m,n,k", [(2, 4096, 4096), (3, 1001, 4112), (4, 33000, 4096),
-                                   (5, 20002, 6144), (7, 3001, 7168), (8, 4099, 8192),
-                                   (6, 517, 8176), (2, 17408, 5120)])
+@pytest.mark.parametrize("m,n,k", QUAD_SHAPES)
 def test_quad_block_kernel(ops, m, n, k):
     """2 <= m <= 4 with 4096 <= K <= 8192, and 5 <= m <= 8 with 5120 < K <= 8192, run the
-    interleaved 4-channel-block kernel: every K range length (4 to 8 units of 64), one
-    and two batch groups, a ragged last K range (4112, 8176), N not a multiple of 4,
-    fewer blocks than CUs, and more blocks per CU than one partial-sum batch holds (N =
-    33000 at one batch group, N = 20002 at two), so the waves also meet mid-way."""
+    interleaved 4-channel-block kernel where the stream kernel is not faster: every K range
+    length (4 to 8 units of 64), one and two batch groups, plain and nontemporal loads, a
+    ragged last K range (4112, 6160, 8176), N not a multiple of 4, fewer blocks than CUs, and
+    more blocks per CU than one partial-sum batch holds (N = 33000 at one batch group, N =
+    20002 at two), so the waves also meet mid-way."""
     rng = np.random.default_rng(m * 11 + n + k)
     x_bits = randn_bf16(rng, (m, k))
     w = rng.integers(-128, 128, (n, k)).astype(np.int8)
@@ -100,17 +109,28 @@ def test_quad_block_kernel(ops, m, n, k):
     check_gemv(bf16_bits(out), x_bits, w, s_bits)
 
 
-@pytest.mark.parametrize("m,n,k", [(1, 5000, 16384), (5, 600, 12288), (8, 300, 12288),
-                                   (16, 70, 9216)])
-def test_long_k_kernels(ops, m, n, k):
-    """K > 8192: x resident in LDS (m * K * 2 <= 64 KiB), the persistent walk over channel
-    blocks (up to 144 KiB) and the LDS ring beyond."""
+@pytest.mark.parametrize("m,n,k", [(12, 1000, 5104), (10, 4100, 5120), (14, 250, 5120),
+                                   (9, 17, 8192), (7, 300, 5120), (5, 2000, 4096),
+                                   (7, 3001, 7168), (8, 4099, 8192)])
+def test_few_channels_per_cu(ops, m, n, k):
+    """M >= 5 with few channels a CU: the stream kernel, one or two 16-channel blocks a tile."""
+    test_balanced_spans(ops, m, n, k)
+
+
+@pytest.mark.parametrize("offset", [0, 2])
+@pytest.mark.parametrize("m,n,k", RESIDENT_SHAPES + [(1, 5000, 16384), (5, 600, 12288),
+                                                     (8, 300, 12288), (16, 70, 9216)])
+def test_long_k_kernels(ops, m, n, k, offset):
+    """K > 8192. x on 16 bytes (offset 0): the stream kernel, but x resident in LDS for
+    RESIDENT_SHAPES. x 4 bytes past 16 (offset 2): resident (m * K * 2 <= 64 KiB: m = 1, 2), the
+    persistent walk over channel blocks (up to 144 KiB: m = 5) and the LDS ring beyond."""
     rng = np.random.default_rng(m * 5 + n + k)
     x_bits = randn_bf16(rng, (m, k))
     w = rng.integers(-128, 128, (n, k)).astype(np.int8)
     s_bits = O.f32_to_bf16(rng.uniform(1e-3, 1e-2, n).astype(np.float32))
     out = torch.full((m, n), float("nan"), device="cuda", dtype=torch.bfloat16)
-    ops.channel_gemv(to_dev(x_bits), to_dev(w), to_dev(s_bits), out)
+    x = to_dev(np.concatenate([np.zeros(offset, np.uint16), x_bits.ravel()]))[offset:].view(m, k)
+    ops.channel_gemv(x, to_dev(w), to_dev(s_bits), out)
     torch.cuda.synchronize()
     check_gemv(bf16_bits(out), x_bits, w, s_bits)
 
