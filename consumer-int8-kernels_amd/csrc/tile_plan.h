@@ -257,27 +257,27 @@ constexpr int kGgufRingThreads = 512;
 
 // Time (us) of the span kernel (gguf_q8.hip, M <= 16) for `channels` of all groups per CU,
 // which it pads to blocks of 16, and K, which its 16 waves' ranges pad to 2, 4, 5 or 8 blocks
-// of 64 each: fitted to 208 shapes measured on MI355X (M = 1..16, N = 1024..8192, K =
-// 1024..8192, one to four groups; rms error 6%). K past 8192 goes in chunks, about 5% more; past
-// 128 channels a CU, which the chunks' partial sums do not fit, the tile kernel takes twice as
-// long (N = 11877, K = 8704, four groups, M = 3: 136 us, the ring 80).
+// of 64 each: fitted to 685 shapes measured on MI355X (M = 1..16, N = 1024..8192, K =
+// 1024..8192, one to four groups; rms error 4%). Rows of whole 128-byte lines take longer. Past
+// 128 channels a CU the partial sums of K's chunks of 8192 do not fit and the tile kernel takes
+// twice as long (N = 11877, K = 8704, four groups, M = 3: 136 us, the ring 80).
 inline double gguf_span_time(int m, int64_t channels, int k) {
-  const int range = (k + 1023) / 1024;
+  const int range = (k + 1023) / 1024, blocks = int((channels + 15) / 16);
   const int held = range <= 2 ? 2 : range <= 4 ? 4 : range <= 5 ? 5 : (range + 7) / 8 * 8;
-  const double time = 2.15 + k / 1024.0 * (0.49 + 0.42 * double(channels) / 16) +
-                      held * (0.027 * m + 0.165 * double((channels + 15) / 16));
-  return k <= 8192 ? time : channels <= 128 ? 1.05 * time : 2 * time;
+  const double time = 2.05 + k / 1024.0 * ((k % 128 ? 0.425 : 0.58) + 0.37 * double(channels) / 16) +
+                      held * (0.0275 * m + 0.192 * blocks + (blocks > 5 ? 0.2 * (blocks - 5) : 0.0));
+  return k > 8192 && blocks > 8 ? 2 * time : time;
 }
 
 // The ring tile for gguf_q8_packed_mm, or -1 where gguf_q8.hip's kernels are expected to be
 // faster: its span kernel up to M = 16, its 256- or 128-row tiles beyond (large_rows, of which
-// it takes the one with fewer rounds). The ring has to be expected 7% below the span kernel,
-// about the models' errors: of those 208 shapes none then ran slower by it than by the span
-// kernel beyond the spread of the runs, and the choice was 0.6% off the best kernel in the mean
-// (N = 7022, K = 1344, M = 12: 4.8 us by the span kernel, 5.7 by the ring; N = 8038, K = 2112,
-// two groups, M = 16 9.6 and 10.4; N = K = 8192, M = 1 21.2 and 14.4); past M = 16 it is 0.3%
-// off over 392. A tile whose workgroups a launch cannot hold (M = 2097120, N = 3, K = 2048, 512
-// groups: 8,388,608 of 128 x 64) is left out.
+// it takes the one with fewer rounds; a 128-row tile of at most 64 rows takes 8% less). The ring
+// has to be expected 3% below the span kernel: of 304 shapes none is then more than 2.5% slower
+// than by the span kernel, and the choice is 0.4% off the best kernel in the mean (N = 7022, K =
+// 1344, M = 12: 4.8 us by the span kernel, 5.7 by the ring; N = 8038, K = 2112, two groups, M = 16
+// 9.6 and 10.4; N = K = 8192, M = 1 21.2 and 14.4); past M = 16 it is 0.3% off over 392. A tile
+// whose workgroups a launch cannot hold (M = 2097120, N = 3, K = 2048, 512 groups: 8,388,608 of
+// 128 x 64) is left out.
 inline int gguf_large_rows(int m, int n, int groups, int cus) {
   const int64_t tiles256 = tile_count(m, n, 256, 128) * groups;
   const int64_t tiles128 = tile_count(m, n, 128, 128) * groups;
@@ -287,11 +287,12 @@ inline int gguf_ring_tile(int m, int n, int k, int groups, int cus) {
   if (cus <= 0) return -1;
   double best;
   if (m <= 16) {
-    best = 0.93 * gguf_span_time(m, (int64_t(n) * groups + cus - 1) / cus, k);
+    best = 0.97 * gguf_span_time(m, (int64_t(n) * groups + cus - 1) / cus, k);
   } else {
     const int rows = gguf_large_rows(m, n, groups, cus);
     best = tiled_time(tile_count(m, n, rows, 128) * groups, cus, rows == 256 ? 8.6 : 4.4,
                       rows == 256 ? 14.2 : 10.7, k);
+    if (m <= 64) best *= 0.92;
   }
   int tile = -1;
   for (int i = 0; i < kGgufTileCount; ++i) {

@@ -14,7 +14,8 @@ sides of the 16-row switch (m <= 16 runs the balanced-span kernel of the W8A16 G
 in chunks of 8192 along K beyond that while a workgroup spans at most 8 channel
 blocks), the 256- and 128-row tiles of larger batches (1, 2, 3, 7 and 8 K
 stages), the 64-row tile kernel that takes x beyond a 2 GiB buffer range, extreme codes
-and scales, and guard sentinels around the output.
+and scales, and guard sentinels around the output. Which kernel a case runs is checked on the
+CPU (tests/test_gpu_gguf_ring.py, whose own cases cover the ring kernel's tiles).
 """
 
 import numpy as np
@@ -89,27 +90,44 @@ def test_reference_cases_with_graph_replay(gguf, m, group_major):
         assert out.float().abs().max() > 0
 
 
-CASES = [
-    # m, groups, n, k, row padding (elements beyond G*K per row)
-    (16, 1, 4096, 4096, 0),     # largest M of the 16-row tile
-    (17, 1, 1000, 5120, 0),     # smallest M past the span kernel, ragged N
+RING_CASES = [
+    # m, groups, n, k, row padding (elements beyond G*K per row); tiles of 16 x 16 or 16 x 32
+    (16, 1, 4096, 4096, 0),
+    (17, 1, 1000, 5120, 0),     # ragged N
     (200, 2, 130, 1536, 64),    # ragged M and N (N % 4 == 2: scalar stores), padded rows
     (64, 4, 96, 64, 8),         # one K stage
-    (5, 2, 37, 16384, 0),       # long K at m <= 16: the span kernel in two K chunks
-    (8, 1, 4096, 14336, 0),     # span kernel, K chunks of 128 and 96 blocks of 64
-    (3, 2, 300, 9216, 64),      # span kernel, a last K chunk of one block per wave
-    (2, 1, 33280, 9216, 0),     # K > 8192 with 9 channel blocks per CU: the tile kernel
+    (8, 1, 4096, 14336, 0),     # long K
+    (5, 2, 37, 16384, 0),
+    (3, 2, 300, 9216, 64),
+    (2, 1, 33280, 9216, 0),     # several tiles per CU
     (256, 1, 512, 2048, 0),
-    (7, 3, 300, 2048, 64),      # m <= 16 span kernel: groups, padded rows, ragged spans
-    (16, 2, 4100, 8192, 0),     # span kernel at its longest K, more channels than CUs x 16
-    (2, 5, 16, 64, 8),          # one channel block per group, one K block
-    # M > 16: 128-channel tiles of 256 or 128 rows (the smaller shapes above run 128 rows)
-    (2048, 1, 4096, 512, 0),    # 256-row tiles, even stage count
-    (1100, 2, 4002, 192, 8),    # 256-row tiles, ragged M, N % 4 == 2, three stages
-    (600, 4, 2000, 448, 24),    # 128-row tiles, ragged M and N, odd stage count
-    (2048, 1, 4096, 64, 0),     # a single K stage
-    (1024, 2, 4096, 128, 0),    # two K stages
 ]
+SPAN_CASES = [
+    (1, 2, 36, 17344, 0),       # long K: three K chunks
+    (1, 1, 4135, 14400, 0),    # more channels than CUs x 16
+    (1, 1, 30, 9024, 64),       # a last K chunk that 13 of the waves have a block of
+    (12, 1, 7022, 1344, 0),     # ragged spans, K ranges of two blocks
+    (3, 1, 6198, 3712, 8),      # of four
+    (1, 1, 6023, 4992, 0),      # of five
+    (7, 3, 300, 2048, 64),      # groups, padded rows, ragged spans
+    (16, 2, 4100, 8192, 0),     # the longest K of one chunk, more channels than CUs x 16
+    (2, 5, 16, 64, 8),          # one channel block per group, one K block
+]
+LARGE_CASES = [
+    # M > 16, 128-channel tiles of 256 rows
+    (256, 2048, 1, 4096, 512, 0),    # even stage count
+    (256, 1100, 2, 4002, 192, 8),    # ragged M, N % 4 == 2, three stages
+    (256, 600, 4, 2000, 448, 24),    # ragged M and N, odd stage count
+    (256, 2048, 1, 4096, 64, 0),     # a single K stage
+    (256, 1024, 2, 4096, 128, 0),    # two K stages
+    # of 128 rows
+    (128, 33, 2, 2063, 64, 0),       # a single K stage, ragged M and N, scalar stores
+    (128, 17, 2, 4770, 128, 8),      # two
+    (128, 17, 3, 5550, 192, 0),      # three, N % 4 == 2
+    (128, 279, 1, 5677, 1024, 8),    # three row tiles, the last ragged
+    (128, 410, 1, 4126, 1024, 0),
+]
+CASES = RING_CASES + SPAN_CASES + [case[1:] for case in LARGE_CASES]
 
 
 @pytest.mark.parametrize("m,groups,n,k,pad", CASES)
@@ -181,7 +199,7 @@ def test_empty_outputs_and_rejections(gguf):
 
 def test_group_major_large_tiles(gguf):
     """x as a group-major view (group stride < row stride is not required: here the
-    group stride is M * K and the row stride K) on the 128-row tiles."""
+    group stride is M * K and the row stride K) on the large tiles."""
     gen = torch.Generator().manual_seed(91)
     m, groups, n, k = 512, 4, 2048, 256
     raw, codes_cpu, scales_cpu = raw_blocks(gen, groups, n, k)
@@ -195,10 +213,11 @@ def test_group_major_large_tiles(gguf):
           scales_cpu.view(torch.int16).numpy().view(np.uint16), rel_norm=0.001)
 
 
-def test_x_beyond_buffer_range_takes_the_tile_kernel(gguf):
-    """A row stride of 2^27 elements puts x's byte range (19 rows x 256 MiB) past what a
-    buffer descriptor addresses, so M = 20 runs the 64-row tile kernel."""
-    m, groups, n, k, xs = 20, 1, 200, 256, 1 << 27
+@pytest.mark.parametrize("m", [12, 20])
+def test_x_beyond_buffer_range_takes_the_tile_kernel(gguf, m):
+    """A row stride of 2^27 elements puts x's byte range (11 or 19 rows x 256 MiB) past what a
+    buffer descriptor addresses, so the calls run the tile kernel of 16 and 64 rows."""
+    groups, n, k, xs = 1, 200, 256, 1 << 27
     rng = np.random.default_rng(5)
     x_np = O.f32_to_bf16(rng.standard_normal((m, groups, k)).astype(np.float32))
     codes_np = rng.integers(-128, 128, (groups, n, k)).astype(np.int8)

@@ -18,7 +18,7 @@ import torch
 from oracle import oracle as O
 from tests.conftest import PKG
 from tests.helpers import bf16_bits, guard_intact, to_dev, with_guard
-from tests.test_gpu_gguf_q8 import check
+from tests.test_gpu_gguf_q8 import LARGE_CASES, RING_CASES, SPAN_CASES, check
 
 SHAPES = [
     # tile, m, groups, n, k, row padding
@@ -37,7 +37,8 @@ int main(int argc, char** argv) {
   for (int i = 1; i + 4 < argc; i += 5) {
     const int t = gguf_ring_tile(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 2]),
                                  atoi(argv[i + 3]), atoi(argv[i + 4]));
-    std::printf("%d %d\n", t < 0 ? 0 : kGgufTiles[t].bm, t < 0 ? 0 : kGgufTiles[t].bn);
+    const int rows = gguf_large_rows(atoi(argv[i]), atoi(argv[i + 1]), atoi(argv[i + 3]), 256);
+    std::printf("%d %d %d\n", t < 0 ? 0 : kGgufTiles[t].bm, t < 0 ? 0 : kGgufTiles[t].bn, rows);
   }
   std::printf("%d\n", kGgufTileCount);
   return 0;
@@ -47,7 +48,8 @@ int main(int argc, char** argv) {
 
 @pytest.fixture(scope="module")
 def choose(tmp_path_factory):
-    """(m, n, k, groups, cus) cases -> chosen (bm, bn), (0, 0) for none; and the tile count."""
+    """(m, n, k, groups, cus) cases -> chosen (bm, bn), (0, 0) for none; the tile count; the rows
+    of the large tiles (gguf_q8.hip) that run the case if it is none and m > 16."""
     gxx = shutil.which("g++")
     if gxx is None:
         pytest.skip("g++ not available")
@@ -59,14 +61,15 @@ def choose(tmp_path_factory):
     def run(cases):
         lines = subprocess.run([str(folder / "plan"), *(str(v) for c in cases for v in c)], check=True,
                                capture_output=True, text=True).stdout.split("\n")
-        return [tuple(map(int, line.split())) for line in lines[: len(cases)]], int(lines[len(cases)])
+        got = [tuple(map(int, line.split())) for line in lines[: len(cases)]]
+        return [g[:2] for g in got], int(lines[len(cases)]), [g[2] for g in got]
 
     return run
 
 
 def test_tile_choices(choose):
     # By hand: M = 2048, N = K = 4096 runs 256 tiles of 256 x 128, one round, 66.9 us, 512
-    # ring tiles of 128 x 128 two of 42.0; M = 1, N = K = 4096 16 channels a CU: 6.6 against
+    # ring tiles of 128 x 128 two of 42.0; M = 1, N = K = 4096 16 channels a CU: 6.7 against
     # 7.5 us for 256 tiles of 16 x 16; without a CU count nothing is chosen.
     # M <= 16 shapes that the span kernel was measured to run up to 19% faster (us, span / ring):
     # 6.8 / 8.1, 4.8 / 5.7, 8.0 / 8.8, 9.0 / 10.1, 9.6 / 10.4, 6.5 / 7.2.
@@ -77,10 +80,21 @@ def test_tile_choices(choose):
     # K > 8192 (us, the other kernels / ring): 135.6 / 80.1, 139.3 / 68.6, 59.7 / 48.9.
     long_k = [(3, 11877, 8704, 4, 256), (1, 8674, 9152, 4, 256), (5, 12024, 9600, 2, 256)]
     assert choose(long_k)[0] == [(16, 32)] * 3
-    got, count = choose(cases)
+    got, count, _ = choose(cases)
     assert got[: len(SHAPES)] == [s[0] for s in SHAPES]
     assert got[len(SHAPES):] == [(0, 0)] * len(by_hand)
     assert len({s[0] for s in SHAPES}) == count
+
+
+def test_cases_of_the_other_kernels(choose):
+    """The cases of test_gpu_gguf_q8.py run the kernels that they are listed under."""
+    got, *_ = choose([(m, n, k, g, 256) for m, g, n, k, _ in RING_CASES])
+    assert (0, 0) not in got
+    got, *_ = choose([(m, n, k, g, 256) for m, g, n, k, _ in SPAN_CASES])
+    assert set(got) == {(0, 0)}
+    got, _, rows = choose([(m, n, k, g, 256) for _, m, g, n, k, _ in LARGE_CASES])
+    assert set(got) == {(0, 0)}
+    assert rows == [case[0] for case in LARGE_CASES]
 
 
 def test_launches_fit_32_bit_work_item_counts(choose):
@@ -89,7 +103,7 @@ def test_launches_fit_32_bit_work_item_counts(choose):
     through small strides) is never chosen, the largest count that fits is."""
     m, n = 65535 * 32, 3
     cases = [(m, n, k, g, 256) for g in (256, 511, 512, 1000, 65535) for k in (64, 1024, 2048, 4096)]
-    got, _ = choose(cases)
+    got, *_ = choose(cases)
     for (*_, groups, _), (bm, bn) in zip(cases, got):
         blocks = -(-m // bm) * -(-n // bn) * groups if bm else 0
         assert blocks * 512 < 2**32, (groups, bm, bn)
