@@ -1225,8 +1225,9 @@ hipError_t dispatch(const int8_t* a, const void* w, const float* sa, const void*
       return launch_ring_gemm(best.ring, a, w, kCode, sa, sw, out, ws, m, n, k, stream);
     case GemmKernel::kPersistent:
       return launch_pp_gemm(a, w, kCode, sa, sw, out, m, n, k, stream);
-    case GemmKernel::kWide256:
-      return run_wlds<WLds256, kCode, kWorkspace>(a, w, sa, sw, out, ws, m, n, k, stream);
+    case GemmKernel::kWide256:  // k % 128 == 0
+      return run_wlds_exact<WLds256, kCode, kWorkspace, true>(a, w, sa, sw, out, ws, m, n, k,
+                                                              stream);
     default:
       return run_wlds<WLds224, kCode, kWorkspace>(a, w, sa, sw, out, ws, m, n, k, stream);
   }

@@ -131,16 +131,22 @@ constexpr int kRingTileCount = sizeof(kRingTiles) / sizeof(kRingTiles[0]);
 // last round that is not full takes three quarters of a round plus its share of the rest
 // (fewer CUs share the caches and the power; the best single share over all tiles).
 constexpr double kLaunchTime = 1.5;
-inline double tiled_time(int64_t tiles, int cus, double fixed, double per_k, int k) {
+inline double tile_rounds(int64_t tiles, int cus) {
   const int64_t rest = tiles % cus;
-  const double rounds = double(tiles / cus) + (rest ? 0.75 + 0.25 * double(rest) / cus : 0.0);
-  return kLaunchTime + rounds * (fixed + per_k * k / 1024);
+  return double(tiles / cus) + (rest ? 0.75 + 0.25 * double(rest) / cus : 0.0);
+}
+inline double tiled_time(int64_t tiles, int cus, double fixed, double per_k, int k) {
+  return kLaunchTime + tile_rounds(tiles, cus) * (fixed + per_k * k / 1024);
 }
 inline int64_t tile_count(int m, int n, int bm, int bn) {
   return int64_t((m + bm - 1) / bm) * ((n + bn - 1) / bn);
 }
+// The ring GEMM's launch; rounds past the first cost it 2% each on all (M = 2696, N = 17148, K =
+// 3232, 6.3 rounds of 192 x 160: 228 us, 200 without).
 inline double ring_time(const RingTile& t, int m, int n, int k, int cus) {
-  return tiled_time(tile_count(m, n, t.bm, t.bn), cus, t.fixed, t.per_k, k);
+  const int64_t tiles = tile_count(m, n, t.bm, t.bn);
+  const double rounds = tile_rounds(tiles, cus);
+  return tiled_time(tiles, cus, t.fixed, t.per_k, k) * (rounds > 1 ? 1 + 0.02 * (rounds - 1) : 1);
 }
 // Widths of the persistent kernel's tiles (256 rows each) with the time of a round, fitted to
 // 122 shapes measured on MI355X (M = 320..16384; (N, K) = 17408 x 5120, 5120 x 17408, 7168 x
@@ -190,14 +196,18 @@ inline double small_time(int m, int n, int k, int cus) {
 // 224-wide tiles (from M = 1024 on; 256 where the persistent kernel can run). cus > 0.
 // workspace: the INT32 products are stored too. out16: the output starts on 16 bytes.
 //
-// The times above are of BF16 outputs whose rows start on 16 bytes. What else costs time grows
-// with the outputs (us per million of them, fitted to 1600 shapes, half with N % 8 == 4 and a
-// third with products):
-//   - the persistent kernel's narrower stores where rows do not start on 16 bytes: 1.7 (M = 1018,
-//     N = 7340, K = 1088: 26.7 us, which a 128 x 128 ring tile does in 18.9);
-//   - the products: 0.85 + 0.03 per 1024 outputs of a ring tile (a round of large tiles stores
-//     them all at its end), 1.1 for the one-wave-per-SIMD kernel, which the ring has to be
-//     expected 10% below there (M = 2870, N = 3716, K = 5088: ring 120 us, that kernel 94).
+// The times above are of BF16 outputs whose rows start on 16 bytes. What else costs time, fitted
+// to 1600 shapes, half with N % 8 == 4 and a third with products, in us:
+//   - the persistent kernel's narrower stores where rows do not start on 16 bytes: 1.0 per
+//     million outputs and 6.5 a round (M = 1018, N = 7340, K = 1088: 26.7, which a 128 x 128 ring
+//     tile does in 18.9);
+//   - the products, per million: 0.85 + 0.03 per 1024 outputs of a ring tile (a round of large
+//     tiles stores them all at its end), 1.1 for the one-wave-per-SIMD kernel, which the ring has
+//     to be expected 10% below there (M = 2870, N = 3716, K = 5088: ring 120, that kernel 94);
+//   - a K tail (K % 128) in 256-wide tiles of that kernel: they take two to three times as long,
+//     so they are left out (M = 1335, N = 10392, K = 9568 with products 403, ring 210; M = 851, N
+//     = 6812, K = 1600 71.6 against 31.5 with 224-wide ones).
+// The choice is 0.8-1.2% off the best kernel in the mean.
 enum class GemmKernel { kSmall, kRing, kPersistent, kWide256, kWide224 };
 struct GemmChoice {
   GemmKernel kernel;
@@ -206,6 +216,7 @@ struct GemmChoice {
 inline GemmChoice gemm_choice(int m, int n, int k, int cus, bool persistent_ok, bool workspace,
                               bool out16 = true) {
   const double outputs = double(m) * n / 1e6;
+  const bool whole_stages = k % 128 == 0;
   GemmChoice ring{GemmKernel::kRing, 0};
   double best = 0.0;
   for (int i = 0; i < kRingTileCount; ++i) {
@@ -226,14 +237,17 @@ inline GemmChoice gemm_choice(int m, int n, int k, int cus, bool persistent_ok, 
     // of 256, 2.69 of 192) 237.8 -> 216.8 us; M = 2048, N = K = 8192 (one round of 256, two of
     // 128, 2% below by the model) measured 118.8 against 124.9, M = 3072, N = 5120, K = 8192
     // (240 of 256, ring 2% below) 112.6 against 119.1.
-    const double time = persistent_time(m, n, k, cus) +
-                        (n % 8 == 0 && out16 ? 0.0 : 1.7 * outputs);
+    double time = persistent_time(m, n, k, cus);
+    if (n % 8 != 0 || !out16) {  // the ring has to be expected 5% below, about the fit's error
+      const int64_t tiles = tile_count(m, n, kPlanBM, pp_width(m, n, k, cus).bn);
+      time = 0.95 * (time + outputs + 6.5 * tile_rounds(tiles, cus));
+    }
     const double wide = 0.95 * wide_time(m, n, kPlanWideBN, k, cus);
-    if (m >= 1024 && !pp_beats_wide_tiles(m, n, cus) && wide <= time)
+    if (whole_stages && m >= 1024 && !pp_beats_wide_tiles(m, n, cus) && wide <= time)
       return wide <= best ? GemmChoice{GemmKernel::kWide256, -1} : ring;
     return time <= best ? GemmChoice{GemmKernel::kPersistent, -1} : ring;
   }
-  const bool wide256 = wide_tiles_pay(m, n, cus);
+  const bool wide256 = whole_stages && wide_tiles_pay(m, n, cus);
   double wide = wide_time(m, n, wide256 ? kPlanWideBN : kPlanBN, k, cus);
   if (workspace) wide = 0.9 * (wide + 1.1 * outputs);
   if (m < 1024 || wide > best) return ring;

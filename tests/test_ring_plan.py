@@ -75,6 +75,15 @@ def test_persistent_widths_have_gpu_shapes(choose):
     assert {width for width, *_ in PP_SHAPES} == {224, 192, 160, 128}
 
 
+def test_256_wide_tiles_take_no_k_tail(choose):
+    """With one they take two to three times as long: 403 us for the second with products, 210 by
+    the ring kernel."""
+    got, _ = choose([(4096, 4096, 1152, 256, "f"), (4096, 4096, 1056, 256, "f"),
+                     (1335, 10392, 9568, 256, "w")])
+    assert got[0] == ("wide", 256, 0)
+    assert got[1][:2] != ("wide", 256) and got[2][0] == "ring"
+
+
 def test_choices_by_hand(choose):
     cases = [
         # M = 4096, N = 17408, K = 5120: 1,248 persistent tiles, 4 + 0.75 + 0.25 * 224 / 256
@@ -96,8 +105,8 @@ def test_choices_by_hand(choose):
         # 0.93 of a round of 157 us, 216 of 192 0.96 of one of 141 us.
         (2048, 5120, 17408, 256, "f"),
         # Rows that do not start on 16 bytes: 232 persistent tiles of 128 take 12.9 us by their
-        # rounds and 12.7 more for 7.5 million outputs, 464 ring tiles of 128 x 128 19.6
-        # (measured: 26.7 us, 18.9).
+        # rounds and 13.6 more for 7.5 million outputs and 0.98 rounds, 464 ring tiles of 128 x
+        # 128 19.6 (measured: 26.7 us, 18.9).
         (1018, 7340, 1088, 256, "f"),
         # With products, 10.7 million outputs: 192 x 128 ring tiles 64 us and 17 for them, 204
         # tiles of 224 in one round 67.7 and 11.7, 10% off (measured: 120 us, 94).
