@@ -237,15 +237,16 @@ def test_down_projection_biased_weights_full_size(ops):
     full_size_check(a_np, w_signed, sa_np, sw_np, ws, out_bits, samples=8)
 
 
+@pytest.mark.parametrize("k", [1152, 1056])
 @pytest.mark.parametrize("biased", [False, True])
-def test_wide_tiles_where_they_fill_the_rounds(ops, biased):
+def test_wide_tiles_where_they_fill_the_rounds(ops, biased, k):
     """M = N = 4096: 304 tiles of 256 x 224 need 2 rounds on 256 CUs and 256 tiles of
     256 x 256 need 1, so schedule 0 (and channel_mm) runs the 256-wide kernel rather than
-    the persistent 224-wide one, with a
-    K that is not a whole number of 128-byte stages. It agrees bit for bit with the
+    the persistent 224-wide one at K = 1152; at K = 1056, not a whole number of 128-byte
+    stages, 256-wide tiles are schedule 3 only. The outputs agree bit for bit with the
     128 x 128 tiling (schedule 1) and, through the exact INT32 accumulators of the
     workspace variant, with the oracle on sampled rows and columns."""
-    m, n, k = 4096, 4096, 1056
+    m, n = 4096, 4096
     rng = np.random.default_rng(256 + biased)
     a_np, w_np, sa_np, sw_np = gemm_inputs(rng, m, n, k, biased=biased)
     w_signed = O.debias(w_np) if biased else w_np
@@ -257,29 +258,39 @@ def test_wide_tiles_where_they_fill_the_rounds(ops, biased):
         ops.fused_channel_mm(a, ws_dev, sa, sw, out, 0)
     ref = torch.empty_like(out)
     ops.fused_channel_mm(a, ws_dev, sa, sw, ref, 1)
+    wide = torch.empty_like(out)
+    ops.fused_channel_mm(a, ws_dev, sa, sw, wide, 3)
     acc = torch.empty(m, n, device="cuda", dtype=torch.int32)
     out2 = torch.empty_like(out)
     ops.cutlass_channel_mm(a, ws_dev, sa, sw, acc, out2)
     torch.cuda.synchronize()
     out_bits = bf16_bits(out)
     assert np.array_equal(out_bits, bf16_bits(ref))
+    assert np.array_equal(out_bits, bf16_bits(wide))
     assert np.array_equal(out_bits, bf16_bits(out2))
     full_size_check(a_np, w_signed, sa_np, sw_np, acc, out_bits, samples=8)
 
 
-@pytest.mark.parametrize("m,n,k,biased", [
-    (2048, 17408, 128, False),   # one K stage: the next tile's copies go out at the switch
-    (2048, 17408, 256, True),    # two stages: group 1 copies the next tile from stage 0
-    (2048, 17408, 384, False),   # an odd stage count: ring slots alternate across tiles
-    (3000, 9000, 1056, True),    # K tail, ragged M and N tiles
-    # On 256 CUs the persistent kernel splits the columns of these: a round of 224-wide
-    # tiles, then one of 160-wide tiles over the rest (tests/test_tile_plan.py checks the
-    # plans), with one K stage, a K tail, a ragged last tile, rows that are not 16-byte
-    # aligned (N = 18500) and ragged M.
-    (1024, 23040, 128, True),
-    (1024, 23040, 640, False),
-    (1100, 18500, 1056, True),
-])
+# Shapes of several tiles per workgroup with the width of the persistent kernel's tiles and, for
+# a column split, the columns of the 224-wide launch before the 160-wide one (256 CUs; checked on
+# the CPU by tests/test_ring_plan.py).
+SWITCHES = [
+    # width, split, m, n, k, biased
+    (192, 0, 2048, 17408, 128, False),  # one K stage: the next tile's copies go out at the switch
+    (192, 0, 2048, 17408, 256, True),   # two stages: group 1 copies the next tile from stage 0
+    (192, 0, 2048, 17408, 384, False),  # an odd stage count: ring slots alternate across tiles
+    (192, 0, 1024, 23040, 128, True),
+    (224, 0, 1025, 19624, 128, False),  # the same, ragged M
+    (224, 0, 1026, 19648, 256, True),
+    (224, 0, 1028, 19616, 384, False),
+    (224, 0, 3000, 9000, 1056, True),   # K tail, ragged M and N tiles
+    (224, 16352, 1537, 20944, 640, False),  # split: ragged M
+    (224, 16352, 1542, 20968, 1056, True),  # and K tail
+    (224, 10304, 2816, 13384, 1056, False),
+]
+
+
+@pytest.mark.parametrize("m,n,k,biased", [case[2:] for case in SWITCHES])
 def test_persistent_tile_switches(ops, m, n, k, biased):
     """Shapes where the persistent kernel runs two or more tiles per workgroup, so each
     workgroup's copy stream runs on from one tile's last stages into the next tile's first
@@ -310,20 +321,18 @@ def test_persistent_tile_switches(ops, m, n, k, biased):
 
 
 @pytest.mark.parametrize("m,n,k,biased", [
-    # 128 < M <= 256 on 256 CUs (tests/test_tile_plan.py checks the choices): 128 x 128
-    # tiles in one round, in 1.5 rounds with a K tail, and at M = 160; 256 x 224 tiles.
     (256, 11264, 256, False),
     (256, 24576, 160, False),
     (160, 16384, 96, True),
     (200, 34816, 128, True),
-    # M >= 1024 with under half the CUs' worth of persistent tiles: 128 x 128 tiles.
     (1024, 2560, 544, True),
     (1100, 2000, 256, False),
 ])
 def test_schedule0_mid_m_and_few_tile_choices(ops, m, n, k, biased):
-    """Schedule 0 where it runs the 128 x 128 or the 256 x 224 kernel in place of the
-    small-M or the persistent kernel. The output equals the 256 x 32 tiling's (schedule 5)
-    and that of the workspace op (which takes the same choice), whose exact INT32
+    """Schedule 0 above the small-M kernel's range and with few large tiles, where it runs narrow
+    persistent or ring tiles, and the 128 x 128 and 256 x 224 tilings that took such shapes
+    once (schedules 1 and 4). The outputs equal the 256 x 32 tiling's (schedule 5)
+    and that of the workspace op, whose exact INT32
     accumulators are checked against the oracle through checksums and sampled rows and
     columns."""
     rng = np.random.default_rng(m * 7 + n + k + biased)
@@ -338,6 +347,11 @@ def test_schedule0_mid_m_and_few_tile_choices(ops, m, n, k, biased):
         ops.fused_channel_mm(a, ws_dev, sa, sw, out, 0)
     ref = torch.empty(m, n, device="cuda", dtype=torch.bfloat16)
     ops.fused_channel_mm(a, ws_dev, sa, sw, ref, 5)
+    for schedule in (1, 4):
+        tiled, tiled_buf = with_guard((m, n), torch.bfloat16, float("nan"))
+        ops.fused_channel_mm(a, ws_dev, sa, sw, tiled, schedule)
+        assert torch.equal(tiled.view(torch.int16), ref.view(torch.int16)), schedule
+        assert guard_intact(tiled_buf, float("nan"))
     acc = torch.empty(m, n, device="cuda", dtype=torch.int32)
     out2 = torch.empty(m, n, device="cuda", dtype=torch.bfloat16)
     ops.cutlass_channel_mm(a, ws_dev, sa, sw, acc, out2)
@@ -349,15 +363,54 @@ def test_schedule0_mid_m_and_few_tile_choices(ops, m, n, k, biased):
     full_size_check(a_np, w_signed, sa_np, sw_np, acc, out_bits, samples=8)
 
 
+# The one-wave-per-SIMD kernel under schedule 0: with INT32 products ("w") or channel scales off
+# 8-byte alignment ("u").
+WIDE_SHAPES = [
+    # width, call, m, n, k
+    (224, "w", 1036, 4484, 256), (224, "w", 1153, 4012, 288), (256, "w", 1025, 11484, 256),
+    (256, "w", 3328, 4272, 256), (224, "u", 1158, 5768, 128), (224, "u", 1153, 5788, 160),
+    (256, "u", 1025, 11484, 256),
+]
+
+
+@pytest.mark.parametrize("width,call,m,n,k", WIDE_SHAPES)
+def test_wide_tiles_with_products_or_unaligned_scales(ops, width, call, m, n, k):
+    """Ragged M and N, K tails, and rows that start on 8 bytes only (N % 8 == 4). The outputs
+    equal the 256 x 32 tiling's (schedule 5), the products the oracle's."""
+    rng = np.random.default_rng(m + n + k + width)
+    a_np, w_np, sa_np, sw_np = gemm_inputs(rng, m, n, k)
+    a, w, sa, sw = to_dev(a_np), to_dev(w_np), to_dev(sa_np), to_dev(sw_np)
+    ref = torch.empty(m, n, device="cuda", dtype=torch.bfloat16)
+    ops.fused_channel_mm(a, w, sa, sw, ref, 5)
+    out, buf = with_guard((m, n), torch.bfloat16, float("nan"))
+    print(f"wide tiles width={width} call={call} m={m} n={n} k={k}", flush=True)
+    if call == "w":
+        acc, acc_buf = with_guard((m, n), torch.int32, -(2**31))
+        ops.cutlass_channel_mm(a, w, sa, sw, acc, out)
+        torch.cuda.synchronize()
+        assert guard_intact(acc_buf, -(2**31))
+        full_size_check(a_np, w_np, sa_np, sw_np, acc, bf16_bits(out), samples=8)
+    else:
+        off = to_dev(np.concatenate([sw_np[:1], sw_np]))[1:]
+        ops.fused_channel_mm(a, w, sa, off, out, 0)
+        biased, biased_buf = with_guard((m, n), torch.bfloat16, float("nan"))
+        ops.channel_mm(a, to_dev(w_np.view(np.uint8) ^ 0x80), sa, off, biased)
+        torch.cuda.synchronize()
+        assert guard_intact(biased_buf, float("nan"))
+        assert np.array_equal(bf16_bits(biased), bf16_bits(ref))
+    assert guard_intact(buf, float("nan"))
+    assert np.array_equal(bf16_bits(out), bf16_bits(ref))
+
+
 @pytest.mark.parametrize("biased", [False, True])
 def test_column_split_in_graph_replays(ops, biased):
     """The column split (a launch of 224-wide tiles over whole rounds, then one of
-    160-wide tiles; M = 1024, N = 23040 on 256 CUs: a round over 14,336 columns, then
-    220 narrow tiles) captured into a HIP graph: three replays, each after eager work that
+    160-wide tiles; M = 1537, N = 20944 on 256 CUs: two rounds over 16,352 columns, then
+    203 narrow tiles over 4,592; the plan is one of SWITCHES) captured into a HIP graph: three replays, each after eager work that
     overwrites the output, equal the eager call bit for bit, and the eager call equals the
     128 x 128 tiling (schedule 1)."""
-    m, n, k = 1024, 23040, 640
-    rng = np.random.default_rng(23040 + biased)
+    m, n, k = 1537, 20944, 640
+    rng = np.random.default_rng(n + biased)
     a_np, w_np, sa_np, sw_np = gemm_inputs(rng, m, n, k, biased=biased)
     w_signed = O.debias(w_np) if biased else w_np
     a, sa, sw, w, ws_dev = to_dev(a_np), to_dev(sa_np), to_dev(sw_np), to_dev(w_np), to_dev(w_signed)

@@ -9,6 +9,7 @@ import subprocess
 import pytest
 
 from tests.conftest import PKG
+from tests.test_gpu_gemm import SWITCHES, WIDE_SHAPES
 from tests.test_gpu_pp_width import SHAPES as PP_SHAPES
 from tests.test_gpu_ring import SHAPES
 
@@ -73,6 +74,18 @@ def test_persistent_widths_have_gpu_shapes(choose):
     got, _ = choose([(m, n, k, 256, "f") for _, m, n, k in PP_SHAPES])
     assert got == [("persistent", width, 0) for width, *_ in PP_SHAPES]
     assert {width for width, *_ in PP_SHAPES} == {224, 192, 160, 128}
+
+
+def test_kernels_of_the_gemm_tests(choose):
+    got, _ = choose([(m, n, k, 256, "f") for _, _, m, n, k, _ in SWITCHES])
+    assert got == [("persistent", width, split) for width, split, *_ in SWITCHES]
+    got, _ = choose([(m, n, k, 256, call) for _, call, m, n, k in WIDE_SHAPES])
+    assert got == [("wide", width, 0) for width, *_ in WIDE_SHAPES]
+    # test_wide_tiles_where_they_fill_the_rounds; the large tilings without their rivals
+    got, _ = choose([(256, 11264, 256, 256, "f"), (200, 34816, 128, 256, "f"),
+                     (1024, 2560, 544, 256, "f")])
+    assert got[0][:2] == ("persistent", 128) and got[1][:2] == ("persistent", 160)
+    assert got[2][0] == "ring"
 
 
 def test_256_wide_tiles_take_no_k_tail(choose):

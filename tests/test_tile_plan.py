@@ -72,7 +72,7 @@ def test_tile_plans(tmp_path):
     assert got[(16384, 5120, 0)] == (0, 0, 0, 0)
     # Fewer tiles than CUs: one round, nothing to split.
     assert got[(1024, 128, 256)] == (0, 224, 0, 1)
-    # The GPU tests' split shapes. 4 x 103 = 412 tiles, the second round 156: one round of
+    # 4 x 103 = 412 tiles, the second round 156: one round of
     # 224-wide tiles over 64 column tiles (14,336 columns), then 8,704 columns as 55 x 4 =
     # 220 narrow tiles: 224 + 180 = 404 < 448 (256-wide: 4 x 90 = 360 tiles, 2 rounds).
     assert got[(1024, 23040, 256)] == (14336, 404, 0, 1)
