@@ -109,17 +109,27 @@ def test_grouped_config5_full_size(ops):
     assert np.array_equal(bf16_bits(out), O.grouped_summed_mm(c_np, s_np, w_np, sw_np))
 
 
-@pytest.mark.parametrize("g,m,n,k", [
-    (3, 1100, 500, 1056),   # ragged M tile, K tail (8.25 stages of 128)
-    (2, 1024, 132, 128),    # one stage per group: copies cross group boundaries at once
-    (1, 1500, 260, 640),    # one group
-    (5, 2048, 256, 256),    # two stages per group
-    (48, 1024, 128, 96),    # the most groups whose row scales fit in LDS, K < one stage
-    (49, 1024, 128, 96),    # one more: the 128 x 128 kernel
+# M >= 1024 shapes that the two-waves-per-SIMD kernel runs (checked on the CPU by
+# tests/test_gpu_grouped_ring.py): its 256 x 128 tiles fill the CUs better than the ring kernel's.
+TWO_WAVES_SHAPES = [
+    (3, 1160, 3224, 544),   # ragged M and N tiles, K tail (4.25 stages of 128)
+    (2, 1032, 3596, 128),   # one stage per group: copies cross group boundaries at once
+    (1, 1028, 3596, 256),   # one group
+    (5, 1156, 3224, 256),   # two stages per group
+    (48, 1672, 1164, 32),   # the most groups whose row scales fit in LDS, K < one stage
+    (1, 2048, 1668, 128),
+]
+
+
+@pytest.mark.parametrize("g,m,n,k", TWO_WAVES_SHAPES + [
+    # shapes of the ring kernel
+    (3, 1100, 500, 1056), (2, 1024, 132, 128), (1, 1500, 260, 640), (5, 2048, 256, 256),
+    (48, 1024, 128, 96), (49, 1024, 128, 96),
 ])
 def test_grouped_large_m_two_waves_per_simd(ops, g, m, n, k):
-    """M >= 1024 (n % 4 == 0) runs the two-waves-per-SIMD kernel over the groups' K stages
-    as one stream; mixed-sign channel scales, guard sentinels and a graph replay."""
+    """M >= 1024 (n % 4 == 0) by the two-waves-per-SIMD kernel over the groups' K stages as one
+    stream, or by the ring kernel; mixed-sign channel scales, guard sentinels and a graph
+    replay."""
     rng = np.random.default_rng(g * 1009 + m + n + k)
     a_np, w_np, sa_np, sw_np = grouped_inputs(rng, g, m, n, k, signed_scales=True)
     a, w, sa, sw = to_dev(a_np), to_dev(w_np), to_dev(sa_np), to_dev(sw_np)
@@ -142,13 +152,17 @@ def test_grouped_large_m_two_waves_per_simd(ops, g, m, n, k):
 @pytest.mark.parametrize("g,m,n,k,sa_offset", [
     (3, 1027, 132, 256, 0),  # m % 4 != 0: groups' row scales not on 16-byte boundaries
     (2, 1024, 132, 256, 1),  # a_scale viewed 4 bytes past a 16-byte boundary
-    (3, 1028, 132, 384, 0),  # m % 4 == 0 and aligned: the two-waves-per-SIMD kernel
+    (3, 1028, 132, 384, 0),
+    (3, 1027, 3600, 384, 0),
+    (3, 1028, 3600, 384, 1),
+    (3, 1028, 3600, 384, 0),  # m % 4 == 0 and aligned: the two-waves-per-SIMD kernel
 ])
 def test_grouped_large_m_row_scale_alignment(ops, g, m, n, k, sa_offset):
-    """The M >= 1024 kernel copies row scales four rows (16 bytes) at a time; shapes and
+    """The two-waves-per-SIMD kernel copies row scales four rows (16 bytes) at a time; shapes and
     a_scale views it cannot copy that way (a copy would straddle a group boundary, be
-    misaligned or run past the end of a_scale) take the row-by-row kernel. Either way the
-    output is the oracle's, bit for bit, including the last group's last rows."""
+    misaligned or run past the end of a_scale) take the ring kernel, which loads them one by
+    one. Either way the output is the oracle's, bit for bit, including the last group's last
+    rows."""
     rng = np.random.default_rng(g * 7919 + m + n + k + sa_offset)
     a_np, w_np, sa_np, sw_np = grouped_inputs(rng, g, m, n, k, signed_scales=True)
     sa_store = torch.full((g * m + sa_offset,), float("nan"), device="cuda")
@@ -157,6 +171,20 @@ def test_grouped_large_m_row_scale_alignment(ops, g, m, n, k, sa_offset):
     assert sa.is_contiguous() and sa.data_ptr() % 16 == 4 * sa_offset % 16
     out, buf = with_guard((m, n), torch.bfloat16, float("nan"))
     ops.grouped_summed_mm(to_dev(a_np), to_dev(w_np), sa, to_dev(sw_np), out)
+    torch.cuda.synchronize()
+    assert np.array_equal(bf16_bits(out), O.grouped_summed_mm(a_np, sa_np, w_np, sw_np))
+    assert guard_intact(buf, float("nan"))
+
+
+@pytest.mark.parametrize("g,m,n,k", [(129, 32, 132, 32), (200, 7, 260, 96), (129, 1, 4, 64),
+                                     (130, 33, 132, 160)])
+def test_grouped_past_the_ring_kernels_row_scales(ops, g, m, n, k):
+    """More groups than a ring tile's LDS holds row scales of (128 at 32 rows): the 32 x 32-MFMA
+    kernel, 256 x 32 tiles up to M = 32 and 128 x 128 tiles above."""
+    rng = np.random.default_rng(g + m + n + k)
+    a_np, w_np, sa_np, sw_np = grouped_inputs(rng, g, m, n, k, signed_scales=True)
+    out, buf = with_guard((m, n), torch.bfloat16, float("nan"))
+    ops.grouped_summed_mm(to_dev(a_np), to_dev(w_np), to_dev(sa_np), to_dev(sw_np), out)
     torch.cuda.synchronize()
     assert np.array_equal(bf16_bits(out), O.grouped_summed_mm(a_np, sa_np, w_np, sw_np))
     assert guard_intact(buf, float("nan"))

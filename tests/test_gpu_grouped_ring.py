@@ -17,7 +17,7 @@ import torch
 from oracle import oracle as O
 from tests.conftest import PKG
 from tests.helpers import bf16_bits, guard_intact, to_dev, with_guard
-from tests.test_gpu_grouped import grouped_inputs
+from tests.test_gpu_grouped import TWO_WAVES_SHAPES, grouped_inputs
 
 SHAPES = [
     # tile, groups, m, n, k
@@ -56,13 +56,16 @@ def test_tile_choices(tmp_path):
     # us; 512 ring tiles of 128 x 128 take 159), which run unless the call rules them out;
     # without a CU count nothing is chosen.
     by_hand = [(2048, 4096, 4096, 4, 256, 1), (2048, 4096, 4096, 4, 256, 0), (64, 4096, 4096, 4, 0, 0)]
-    cases = [(m, n, k, g, 256, 0) for _, g, m, n, k in SHAPES] + by_hand
+    two_waves = [(m, n, k, g, 256, 1) for g, m, n, k in [*TWO_WAVES_SHAPES, (3, 1028, 3600, 384)]]
+    cases = [(m, n, k, g, 256, 0) for _, g, m, n, k in SHAPES] + by_hand + two_waves
     lines = subprocess.run([str(tmp_path / "plan"), *(str(v) for c in cases for v in c)], check=True,
                            capture_output=True, text=True).stdout.split("\n")
     got = [tuple(map(int, line.split())) for line in lines[: len(cases)]]
     assert got[: len(SHAPES)] == [s[0] for s in SHAPES]
     assert got[len(SHAPES)] == (0, 0) and got[len(SHAPES) + 1] != (0, 0)
     assert got[len(SHAPES) + 2] == (0, 0)
+    assert got[len(SHAPES) + len(by_hand):] == [(0, 0)] * len(two_waves)
+    assert all(m >= 1024 and m % 4 == 0 and n % 4 == 0 for m, n, *_ in two_waves)
     assert len({s[0] for s in SHAPES} - {(0, 0)}) == int(lines[len(cases)])
 
 
