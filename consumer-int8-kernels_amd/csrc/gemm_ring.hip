@@ -10,8 +10,8 @@
 // the ring's depth (3 to 8 slots), the number of busy CUs (64 to 256), the cache policy of
 // the copies or an L2 prefetch of the panels by a ninth wave (all measured within 3%; the
 // nontemporal policy 10-50% slower). So the tile is picked per shape (tile_plan.h) to put
-// one tile on every CU with as few operand bytes as possible, instead of splitting K over
-// workgroups, whose INT32 partials would move as many bytes as they save.
+// one tile on every CU with as few operand bytes as possible. (Splitting K over workgroups would
+// copy fewer, but the entry points have no buffer for the partial sums and no counter.)
 //
 // Measured on MI355X against the kernels that took these shapes before (fused_channel_mm
 // alone, three rotated weight copies, identical outputs), us: M = 256, N = 7168, K = 5120:
