@@ -142,11 +142,13 @@ inline int64_t tile_count(int m, int n, int bm, int bn) {
   return int64_t((m + bm - 1) / bm) * ((n + bn - 1) / bn);
 }
 // The ring GEMM's launch; rounds past the first cost it 2% each on all (M = 2696, N = 17148, K =
-// 3232, 6.3 rounds of 192 x 160: 228 us, 200 without).
+// 3232, 6.3 rounds of 192 x 160: 228 us, 200 without). Below K = 1024 a round's fixed part shrinks,
+// down to 70% (M = 10, N = 24936, K = 96 by 64 x 128 tiles: 3.96 us, 5.0 without).
 inline double ring_time(const RingTile& t, int m, int n, int k, int cus) {
   const int64_t tiles = tile_count(m, n, t.bm, t.bn);
   const double rounds = tile_rounds(tiles, cus);
-  return tiled_time(tiles, cus, t.fixed, t.per_k, k) * (rounds > 1 ? 1 + 0.02 * (rounds - 1) : 1);
+  const double fixed = t.fixed * (k < 1024 ? 0.7 + 0.3 * k / 1024 : 1.0);
+  return tiled_time(tiles, cus, fixed, t.per_k, k) * (rounds > 1 ? 1 + 0.02 * (rounds - 1) : 1);
 }
 // Widths of the persistent kernel's tiles (256 rows each) with the time of a round, fitted to
 // 122 shapes measured on MI355X (M = 320..16384; (N, K) = 17408 x 5120, 5120 x 17408, 7168 x
@@ -184,10 +186,13 @@ inline double persistent_time(int m, int n, int k, int cus) {
 inline double wide_time(int m, int n, int bn, int k, int cus) {
   return tiled_time(tile_count(m, n, kPlanBM, bn), cus, 9.7, 13.8 * bn / kPlanWideBN, k);
 }
+// The small-M kernel's launch: its rounds' fixed part grows with the tile as well, fitted to 638
+// shapes (M <= 512, K = 32..16384; rms error 9%): M = 43, N = 928, K = 288 (174 tiles of 16 x 16)
+// 2.4 us, the ring's best tile 3.6.
 inline double small_time(int m, int n, int k, int cus) {
   const SmallShape s = small_best_shape(m, n, cus);
   const double rounds = double((tile_count(m, n, s.bm, s.bn) + cus - 1) / cus);
-  return kLaunchTime + rounds * (2.05 + 0.01146 * (s.bm + s.bn) * k / 1024);
+  return kLaunchTime + rounds * (s.bm + s.bn) * (0.019 + 0.012 * k / 1024);
 }
 
 // Schedule 0's kernel, by the times above: the ring kernel with tile kRingTiles[ring] where that
@@ -202,12 +207,13 @@ inline double small_time(int m, int n, int k, int cus) {
 //     million outputs and 6.5 a round (M = 1018, N = 7340, K = 1088: 26.7, which a 128 x 128 ring
 //     tile does in 18.9);
 //   - the products, per million: 0.85 + 0.03 per 1024 outputs of a ring tile (a round of large
-//     tiles stores them all at its end), 1.1 for the one-wave-per-SIMD kernel, which the ring has
-//     to be expected 10% below there (M = 2870, N = 3716, K = 5088: ring 120, that kernel 94);
-//   - a K tail (K % 128) in 256-wide tiles of that kernel: they take two to three times as long,
-//     so they are left out (M = 1335, N = 10392, K = 9568 with products 403, ring 210; M = 851, N
-//     = 6812, K = 1600 71.6 against 31.5 with 224-wide ones).
-// The choice is 0.8-1.2% off the best kernel in the mean.
+//     tiles stores them all at its end), 1.3 for the one-wave-per-SIMD kernel, which the ring has
+//     to be expected 5% below there (M = 2870, N = 3716, K = 5088: ring 120, that kernel 94);
+//   - a K tail (K % 128) in 256-wide tiles of that kernel: it spills 174 registers a lane and
+//     takes 2.8 times as long, so they are left out (M = 1335, N = 10392, K = 9568 with products
+//     403, ring 210; M = 851, N = 6812, K = 1600 71.6 against 31.5 with 224-wide ones).
+// The choice is 0.8-1.1% off the best kernel in the mean from K = 1024 on, and below 0.4% up to M
+// = 256 and 2-4% beyond.
 enum class GemmKernel { kSmall, kRing, kPersistent, kWide256, kWide224 };
 struct GemmChoice {
   GemmKernel kernel;
@@ -225,8 +231,8 @@ inline GemmChoice gemm_choice(int m, int n, int k, int cus, bool persistent_ok, 
     if (workspace) t += outputs * (0.85 + 0.03 * tile.bm * tile.bn / 1024);
     if (i == 0 || t < best) best = t, ring.ring = i;
   }
-  // The ring has to be expected 3% below the small-M kernel: level by the times, it was 5-7%
-  // slower at the smallest calls (M = 186, N = 1496, K = 1312: 4.86 us against 4.60).
+  // The ring has to be expected 3% below the small-M kernel: level by the times, it was 4% or more
+  // slower at 13 of 293 shapes below K = 1024, and is at 6.
   if (m <= kSmallMaxM &&
       0.97 * (small_time(m, n, k, cus) + (workspace ? 0.85 * outputs : 0.0)) <= best)
     return {GemmKernel::kSmall, -1};
@@ -249,7 +255,7 @@ inline GemmChoice gemm_choice(int m, int n, int k, int cus, bool persistent_ok, 
   }
   const bool wide256 = whole_stages && wide_tiles_pay(m, n, cus);
   double wide = wide_time(m, n, wide256 ? kPlanWideBN : kPlanBN, k, cus);
-  if (workspace) wide = 0.9 * (wide + 1.1 * outputs);
+  if (workspace) wide = 0.95 * (wide + 1.3 * outputs);
   if (m < 1024 || wide > best) return ring;
   return {wide256 ? GemmKernel::kWide256 : GemmKernel::kWide224, -1};
 }

@@ -280,8 +280,8 @@ SWITCHES = [
     (192, 0, 2048, 17408, 256, True),   # two stages: group 1 copies the next tile from stage 0
     (192, 0, 2048, 17408, 384, False),  # an odd stage count: ring slots alternate across tiles
     (192, 0, 1024, 23040, 128, True),
-    (224, 0, 1025, 19624, 128, False),  # the same, ragged M
-    (224, 0, 1026, 19648, 256, True),
+    (224, 0, 781, 24592, 128, False),  # the same, ragged M
+    (224, 0, 770, 24624, 256, True),
     (224, 0, 1028, 19616, 384, False),
     (224, 0, 3000, 9000, 1056, True),   # K tail, ragged M and N tiles
     (224, 16352, 1537, 20944, 640, False),  # split: ragged M
@@ -367,8 +367,8 @@ def test_schedule0_mid_m_and_few_tile_choices(ops, m, n, k, biased):
 # 8-byte alignment ("u").
 WIDE_SHAPES = [
     # width, call, m, n, k
-    (224, "w", 1036, 4484, 256), (224, "w", 1153, 4012, 288), (256, "w", 1025, 11484, 256),
-    (256, "w", 3328, 4272, 256), (224, "u", 1158, 5768, 128), (224, "u", 1153, 5788, 160),
+    (224, "w", 1036, 7228, 256), (224, "w", 1041, 7332, 288), (256, "w", 1025, 11484, 256),
+    (256, "w", 3328, 4272, 256), (224, "u", 1755, 5812, 128), (224, "u", 1166, 8236, 160),
     (256, "u", 1025, 11484, 256),
 ]
 

@@ -13,7 +13,7 @@ from tests import test_gpu_ring
 pytestmark = pytest.mark.gpu
 
 SHAPES = [
-    (128, 609, 3208, 32), (128, 2592, 9240, 32), (128, 1556, 9240, 128), (128, 1038, 6024, 416),
+    (128, 653, 6760, 32), (128, 2592, 9240, 32), (128, 1556, 9240, 128), (128, 1038, 6024, 416),
     (160, 769, 8368, 32), (160, 772, 8352, 128), (160, 2592, 6024, 160),
     (160, 1297, 6024, 1056), (192, 2592, 12456, 32), (192, 775, 10408, 128),
     (192, 2333, 4416, 160), (192, 1038, 9240, 1056), (224, 769, 12344, 128),
