@@ -372,8 +372,11 @@ inline int grouped_ring_tile(int m, int n, int k, int groups, int cus, bool pers
 //     32.0; 2128 x 14688: 10.0 against 9.6, 26801 x 9280: 55.1 against 47.2).
 //   M >= 5, up to 16 channels a CU: with lines everywhere (4096 x 4096: 6.2-6.6 against 7.5-8.3).
 //     Without, from K = 2048 on, at M <= 7 up to K = 7168 (2481 x 7824, M = 5: 8.7 against 8.2),
-//     and below where rows are whole half lines (1866 x 1984, M = 8: 3.5 against 3.7; otherwise 31
-//     of 71 shapes ran 2-8% slower: 1684 x 1040, M = 10 3.4 against 3.1).
+//     at M <= 6 and four channels a CU up to 5120 (586 x 5776, M = 6: 5.4 against 4.6); below K =
+//     2048 where rows are whole half lines (1866 x 1984, M = 8: 3.5 against 3.7; otherwise 31
+//     of 71 shapes ran 2-8% slower: 1684 x 1040, M = 10 3.4 against 3.1) and below K = 1024 (3622 x
+//     80, M = 16: 2.7 against 3.0; 366 x 944: 2.9 against 3.1), there up to 20 channels a CU (4373
+//     x 16, M = 10: 2.9 against 3.3).
 //   17 to 20 channels a CU (24 computed): with lines up to 19, or from K = 5120 on (5120 x 5120:
 //     8.2-9.4 against 8.5-10.9; 5036 x 3456, M = 9: 7.8 against 7.5); without, M >= 13 from 18
 //     channels and K = 5120 on (5047 x 5568, M = 14: 10.4 against 11.7; 4839 x 1808, M = 14: 5.6
@@ -409,7 +412,11 @@ inline bool gemv_stream_pays(int m, int64_t channels, int n, int k) {
            !(channels > 24 && channels <= 32 && k < 12000);
   }
   if (m < 5) return false;
-  if (channels <= 16) return lines || (k >= 2048 ? m >= 8 || k < 7168 : k % 64 == 0);
+  if (channels <= 16 || (channels <= 20 && k < 1024)) {
+    if (lines) return true;
+    if (k < 2048) return k < 1024 || k % 64 == 0;
+    return m >= 8 || k < (m <= 6 && channels <= 4 ? 5120 : 7168);
+  }
   if (lines && (channels <= 19 || (channels <= 20 && k >= 5120))) return true;
   return channels <= 40 && k >= 5120 && (lines ? m >= 9 : m >= 13 && channels >= 18);
 }

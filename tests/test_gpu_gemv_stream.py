@@ -25,6 +25,7 @@ SHAPES = [
     (3, 6, 4861, 256), (3, 16, 4864, 2176), (4, 13, 8190, 5136), (5, 12, 10001, 5120),
     (6, 1, 12003, 8320), (7, 3, 14001, 8208), (8, 4, 16001, 8208), (9, 2, 18001, 8208),
     (5, 7, 19000, 8224), (3, 4, 5120, 17408),
+    (1, 5, 999, 16), (2, 16, 3622, 80), (1, 8, 366, 944),
     # past 96 MB: nontemporal copies
     (7, 9, 27001, 4096), (6, 5, 24501, 4224), (5, 16, 18433, 8192), (9, 12, 34817, 3072 + 1152), (6, 1, 11801, 8576),
 ]
@@ -57,11 +58,13 @@ def test_choices(tmp_path):
               (1, 26801, 9280, 256), (1, 3755, 8832, 256), (2, 7846, 9984, 256),
               (10, 1684, 1040, 256), (5, 2481, 7824, 256), (14, 4839, 1808, 256),
               (9, 5000, 1616, 256), (11, 8630, 7056, 256), (8, 5102, 6416, 256),
-              (9, 5036, 3456, 256),
+              (9, 5036, 3456, 256), (6, 586, 5776, 256), (5, 129, 7584, 256),
               *((*s, 256) for s in SPAN_SHAPES + QUAD_SHAPES + RESIDENT_SHAPES)]
     # measured up to 12% faster on it
     taken = [(14, 5047, 5568, 256), (8, 1866, 1984, 256), (2, 6352, 17408, 256),
-             (1, 6352, 17408, 256), (1, 5120, 17408, 256), (3, 2088, 9712, 256)]
+             (1, 6352, 17408, 256), (1, 5120, 17408, 256), (3, 2088, 9712, 256),
+             (16, 366, 944, 256), (8, 924, 6480, 256),
+             (10, 4373, 16, 256)]
     cases = [(m, n, k, 256) for _, m, n, k in SHAPES] + others + taken
     lines = subprocess.run([str(tmp_path / "plan"), *(str(v) for c in cases for v in c)], check=True,
                            capture_output=True, text=True).stdout.split()
