@@ -295,7 +295,10 @@ inline double gguf_span_time(int m, int64_t channels, int k) {
 // has to be expected 3% below the span kernel: of 304 shapes none is then more than 2.5% slower
 // than by the span kernel, and the choice is 0.4% off the best kernel in the mean (N = 7022, K =
 // 1344, M = 12: 4.8 us by the span kernel, 5.7 by the ring; N = 8038, K = 2112, two groups, M = 16
-// 9.6 and 10.4; N = K = 8192, M = 1 21.2 and 14.4); past M = 16 it is 0.3% off over 392. A tile
+// 9.6 and 10.4; N = K = 8192, M = 1 21.2 and 14.4); past M = 16 it is 0.3% off over 392. At M <=
+// 16, K <= 1024 and up to 16 channels a CU, where launch and latency are most of both, the ring's
+// 16 x 16 tiles are faster up to K = 256, one stage, and the span kernel beyond, at each of 170
+// shapes (N = 520, M = 2, K = 256 3.01 us and 3.23; N = 502, M = 14, K = 320 3.68 and 3.35). A tile
 // whose workgroups a launch cannot hold (M = 2097120, N = 3, K = 2048, 512 groups: 8,388,608 of
 // 128 x 64) is left out.
 inline int gguf_large_rows(int m, int n, int groups, int cus) {
@@ -307,7 +310,9 @@ inline int gguf_ring_tile(int m, int n, int k, int groups, int cus) {
   if (cus <= 0) return -1;
   double best;
   if (m <= 16) {
-    best = 0.97 * gguf_span_time(m, (int64_t(n) * groups + cus - 1) / cus, k);
+    const int64_t channels = (int64_t(n) * groups + cus - 1) / cus;
+    if (k <= 1024 && channels <= 16) return k <= 256 ? 0 : -1;
+    best = 0.97 * gguf_span_time(m, channels, k);
   } else {
     const int rows = gguf_large_rows(m, n, groups, cus);
     best = tiled_time(tile_count(m, n, rows, 128) * groups, cus, rows == 256 ? 8.6 : 4.4,

@@ -96,6 +96,7 @@ RING_CASES = [
     (17, 1, 1000, 5120, 0),     # ragged N
     (200, 2, 130, 1536, 64),    # ragged M and N (N % 4 == 2: scalar stores), padded rows
     (64, 4, 96, 64, 8),         # one K stage
+    (2, 5, 16, 64, 8),
     (8, 1, 4096, 14336, 0),     # long K
     (5, 2, 37, 16384, 0),
     (3, 2, 300, 9216, 64),
@@ -111,7 +112,8 @@ SPAN_CASES = [
     (1, 1, 6023, 4992, 0),      # of five
     (7, 3, 300, 2048, 64),      # groups, padded rows, ragged spans
     (16, 2, 4100, 8192, 0),     # the longest K of one chunk, more channels than CUs x 16
-    (2, 5, 16, 64, 8),          # one channel block per group, one K block
+    (2, 5, 16, 320, 8),         # one channel block per group, five K blocks for 16 waves
+    (2, 5, 868, 64, 8),         # one K block
 ]
 LARGE_CASES = [
     # M > 16, 128-channel tiles of 256 rows

@@ -72,14 +72,18 @@ def test_tile_choices(choose):
     # ring tiles of 128 x 128 two of 42.0; M = 1, N = K = 4096 16 channels a CU: 6.7 against
     # 7.5 us for 256 tiles of 16 x 16; without a CU count nothing is chosen.
     # M <= 16 shapes that the span kernel was measured to run up to 19% faster (us, span / ring):
-    # 6.8 / 8.1, 4.8 / 5.7, 8.0 / 8.8, 9.0 / 10.1, 9.6 / 10.4, 6.5 / 7.2.
+    # 6.8 / 8.1, 4.8 / 5.7, 8.0 / 8.8, 9.0 / 10.1, 9.6 / 10.4, 6.5 / 7.2, 3.35 / 3.68.
     span = [(2, 3437, 3136, 2, 256), (12, 7022, 1344, 1, 256), (3, 6198, 3712, 1, 256),
-            (1, 6023, 4992, 1, 256), (16, 8038, 2112, 2, 256), (6, 8168, 2240, 1, 256)]
+            (1, 6023, 4992, 1, 256), (16, 8038, 2112, 2, 256), (6, 8168, 2240, 1, 256),
+            (14, 502, 320, 1, 256)]
     by_hand = [(2048, 4096, 4096, 1, 256), (1, 4096, 4096, 1, 256), (64, 4096, 4096, 1, 0), *span]
     cases = [(m, n, k, g, 256) for _, m, g, n, k, _ in SHAPES] + by_hand
     # K > 8192 (us, the other kernels / ring): 135.6 / 80.1, 139.3 / 68.6, 59.7 / 48.9.
     long_k = [(3, 11877, 8704, 4, 256), (1, 8674, 9152, 4, 256), (5, 12024, 9600, 2, 256)]
     assert choose(long_k)[0] == [(16, 32)] * 3
+    # One K stage, up to 16 channels a CU: 3.23 / 3.01, 3.42 / 3.06, 3.21 / 3.06.
+    short_k = [(2, 520, 256, 1, 256), (3, 3532, 256, 1, 256), (10, 200, 64, 2, 256)]
+    assert choose(short_k)[0] == [(16, 16)] * 3
     got, count, _ = choose(cases)
     assert got[: len(SHAPES)] == [s[0] for s in SHAPES]
     assert got[len(SHAPES):] == [(0, 0)] * len(by_hand)
