@@ -280,13 +280,18 @@ constexpr int kGgufRingThreads = 512;
 // of 64 each: fitted to 685 shapes measured on MI355X (M = 1..16, N = 1024..8192, K =
 // 1024..8192, one to four groups; rms error 4%). Rows of whole 128-byte lines take longer. Past
 // 128 channels a CU the partial sums of K's chunks of 8192 do not fit and the tile kernel takes
-// twice as long (N = 11877, K = 8704, four groups, M = 3: 136 us, the ring 80).
+// twice as long (N = 11877, K = 8704, four groups, M = 3: 136 us, the ring 80). Past 64 channels a
+// CU with ranges past 4 blocks the fit is 18% short up to M = 8 (N = 8078, K = 7168, four groups,
+// M = 2: 51.5 us for 44.2, the ring 45.5); beyond, the ring is the one that is short (M = 12, N =
+// 7257, K = 7488: 51.1, the ring 55.8).
 inline double gguf_span_time(int m, int64_t channels, int k) {
   const int range = (k + 1023) / 1024, blocks = int((channels + 15) / 16);
   const int held = range <= 2 ? 2 : range <= 4 ? 4 : range <= 5 ? 5 : (range + 7) / 8 * 8;
-  const double time = 2.05 + k / 1024.0 * ((k % 128 ? 0.425 : 0.58) + 0.37 * double(channels) / 16) +
-                      held * (0.0275 * m + 0.192 * blocks + (blocks > 5 ? 0.2 * (blocks - 5) : 0.0));
-  return k > 8192 && blocks > 8 ? 2 * time : time;
+  const double time =
+      2.05 + k / 1024.0 * ((k % 128 ? 0.425 : 0.58) + 0.37 * double(channels) / 16) +
+      held * (0.0275 * m + 0.192 * blocks + (blocks > 5 ? 0.2 * (blocks - 5) : 0.0));
+  if (k > 8192) return blocks > 8 ? 2 * time : time;
+  return blocks > 4 && range > 4 && m <= 8 ? 1.18 * time : time;
 }
 
 // The ring tile for gguf_q8_packed_mm, or -1 where gguf_q8.hip's kernels are expected to be

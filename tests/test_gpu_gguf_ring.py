@@ -84,6 +84,10 @@ def test_tile_choices(choose):
     # One K stage, up to 16 channels a CU: 3.23 / 3.01, 3.42 / 3.06, 3.21 / 3.06.
     short_k = [(2, 520, 256, 1, 256), (3, 3532, 256, 1, 256), (10, 200, 64, 2, 256)]
     assert choose(short_k)[0] == [(16, 16)] * 3
+    # 64 and more channels a CU: 51.5 / 45.5, 47.0 / 43.2, 46.7 / 42.4; past M = 8 51.1 / 55.8, 33.9 / 36.2.
+    many = [(2, 8078, 7168, 4, 256), (5, 7284, 6912, 4, 256), (3, 4029, 5824, 8, 256),
+            (12, 7257, 7488, 4, 256), (16, 5339, 5952, 4, 256)]
+    assert choose(many)[0] == [(16, 32)] * 3 + [(0, 0)] * 2
     got, count, _ = choose(cases)
     assert got[: len(SHAPES)] == [s[0] for s in SHAPES]
     assert got[len(SHAPES):] == [(0, 0)] * len(by_hand)
